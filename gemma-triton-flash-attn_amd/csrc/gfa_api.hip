@@ -134,6 +134,33 @@ gfa::QGrid make_qgrid(int B, int Hkv, int R, int N, int nu) {
   return g;
 }
 
+// The forward kernel for small grids (gfa_fwd_rows.hip: one workgroup per 32 query rows, its
+// waves splitting the keys) where fwd_kernel's 128-row workgroups leave CUs idle and its time is
+// the longest row's serial walk. Counted in 32-row blocks, one resident workgroup per CU:
+// - up to 256 (one round): 1.5-1.6x faster at D=512 (8:1 N=1024 causal 50.7 -> 31.5 us), up to
+//   1.8x at D=256 and below (8:4 D=256 N=1024 30.0 -> 16.7 us). At D=64 a sequence of up to one
+//   128-key tile has nothing to split (5.2 -> 5.8 us) and stays;
+// - up to 512 under full causal masking, whose second round is the short rows: D=512 8:1 N=2048
+//   90.7 -> 71.3, D=256 8:4 N=2048 54.1 -> 34.1, D=128 8:2 N=2048 35.4 -> 22.0 us; below D=256
+//   only from 1024 tokens (D=128 32:8 N=333 10.6 -> 11.8 us).
+// Past that the K / V copies per 32 rows cost more than the idle CUs (D=512 8:1 N=3000, 752
+// blocks: 128 -> 142 us; windows: D=256 8:1 W=512 N=1500, 376 blocks: 20.2 -> 23.5 us).
+bool use_rows_kernel(int D, int B, int Hq, int N, bool causal, bool windowed) {
+  const long long blocks = (long long)B * Hq * ((N + 31) / 32);
+  if (D == 64 && N <= 128) return false;
+  if (blocks <= 256) return true;
+  return blocks <= 512 && causal && !windowed && (D >= 256 || N >= 1024);
+}
+
+gfa::QGrid rows_grid(int B, int Hkv, int R, int N) {
+  gfa::QGrid g;
+  g.hpw = g.qbw = 1;
+  g.n_hg = R;
+  g.n_qsb = (N + 31) / 32;
+  g.nblocks = g.n_qsb * B * Hkv * R;
+  return g;
+}
+
 // Smallest of {1, 2, 4, 8} that fills the GPU with dK/dV workgroups: `rounds` rounds of
 // 256 CUs x wgs_per_cu resident workgroups. A full-causal grid needs two rounds: its key
 // blocks carry unequal work, which the heaviest-first grid order balances once there are
@@ -158,8 +185,9 @@ gfa::RowView rv(const gfa_strides& s) { return gfa::RowView{s.batch, s.head, s.r
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Rows past the end of a slice that a tile copy may address (largest tile 64 rows, and a
-// loop's last prefetch starts at most one tile past the last row).
+// Rows past the end of a slice that a tile copy may address: the largest tiles are 64 rows with a
+// last prefetch that starts at most one tile past the last row, and 128 rows (gfa_fwd_rows.hip)
+// that start at row N at most.
 constexpr int kTileOverrun = 128;
 
 int check_view(const char* name, const void* ptr, const gfa_strides& s, bool need_ptr) {
@@ -389,6 +417,13 @@ int gfa_fwd(const gfa_fwd_args* a) {
   if (p.store_lse && (a->lse_ld < GFA_LSE_LD(a->seq_len) || !aligned16(a->lse) || (a->lse_ld & 3)))
     return fail(GFA_ERR_INVALID_ARGUMENT, "lse_ld=%d must be >= %d (multiple of 4, 16-byte aligned lse)", a->lse_ld,
                 GFA_LSE_LD(a->seq_len));
+  if (a->block_kv == 0 && use_rows_kernel(a->head_dim, p.B, p.Hq, p.N, p.causal, windowed)) {
+    p.g = rows_grid(p.B, p.Hkv, p.R, p.N);
+    const hipError_t err = gfa::launch_fwd_rows(p, a->head_dim, a->dtype == GFA_DTYPE_BF16, cap, drop,
+                                                static_cast<hipStream_t>(a->stream));
+    if (err != hipSuccess) return fail(GFA_ERR_LAUNCH, "forward launch failed: %s", hipGetErrorString(err));
+    return ok();
+  }
   p.g = make_qgrid(p.B, p.Hkv, p.R, p.N, nw);
   if (p.g.nblocks <= 0) return fail(GFA_ERR_INVALID_ARGUMENT, "empty grid");
   if ((rc = setup_queue(static_cast<hipStream_t>(a->stream), a->head_dim, p.g.nblocks, &p.sched))) return rc;

@@ -7,6 +7,7 @@ namespace gfa {
 
 hipError_t launch_fwd(const FwdParams& p, int head_dim, int block_kv, int nwaves, bool bf16, bool cap, bool drop,
                       hipStream_t stream);
+hipError_t launch_fwd_rows(const FwdParams& p, int head_dim, bool bf16, bool cap, bool drop, hipStream_t stream);
 hipError_t launch_bwd_dq(const BwdDqParams& p, int head_dim, int block_kv, int split, bool bf16, bool cap, bool drop,
                          hipStream_t stream);
 hipError_t launch_bwd_dkv(const BwdDkvParams& p, int head_dim, int block_q, int waves, int roles, bool bf16, bool cap,

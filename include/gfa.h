@@ -87,7 +87,8 @@ typedef struct {
   int32_t window;      /* sliding window; 0 = off; honoured only when causal; >= seq_len -> off */
   float scale;         /* softmax scale, finite and > 0; the reference uses 1/sqrt(head_dim) */
   int32_t dtype;       /* gfa_dtype, shared by q/k/v/o */
-  int32_t block_kv;    /* 0 = registry default, else a built tile width */
+  int32_t block_kv;    /* 0 = library's choice (the registry's tile; small grids run a kernel that
+                          splits the keys over a workgroup's waves), else a built tile width */
   int32_t lse_ld;      /* row length of lse (>= GFA_LSE_LD(seq_len)); ignored when lse == NULL */
   void* stream;        /* hipStream_t */
   const int32_t* seg_lo; /* optional (B, N) segment table (see above); NULL = one segment per row */
