@@ -33,10 +33,11 @@ STATUS_NAMES = {
 # GFA_VERSION of include/gfa.h whose struct layouts FwdArgs / BwdArgs below mirror. A library
 # built from other sources reads another prefix of the argument structs (an older one ignores the
 # segment, soft-cap and dropout fields), so load() refuses it instead of computing wrong results.
-ABI_VERSION = 106
+ABI_VERSION = 107
 
 EXPORTED = ("gfa_fwd", "gfa_bwd", "gfa_bwd_noalloc", "gfa_bwd_workspace_size", "gfa_bwd_workspace_bytes",
-            "gfa_bwd_ds_limit", "gfa_config", "gfa_last_error", "gfa_version", "gfa_set_runtime_scheduling")
+            "gfa_bwd_ds_limit", "gfa_config", "gfa_last_error", "gfa_version", "gfa_set_runtime_scheduling",
+            "gfa_segments_from_positions", "gfa_segments_from_mask")
 NOALLOC_SCRATCH_BYTES = 64 << 20  # GFA_NOALLOC_SCRATCH_BYTES
 
 
@@ -131,6 +132,11 @@ def load() -> ctypes.CDLL:
         lib.gfa_version.restype = ctypes.c_int
         lib.gfa_set_runtime_scheduling.argtypes = [ctypes.c_int32]
         lib.gfa_set_runtime_scheduling.restype = ctypes.c_int
+        ptr, i32, i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
+        lib.gfa_segments_from_positions.argtypes = [ptr, i32, i64, i32, i32, ptr, ptr, ptr]
+        lib.gfa_segments_from_positions.restype = ctypes.c_int
+        lib.gfa_segments_from_mask.argtypes = [ptr, i64, i32, i32, ptr, ptr, ptr, ptr]
+        lib.gfa_segments_from_mask.restype = ctypes.c_int
         built = int(lib.gfa_version())
         if built != ABI_VERSION:
             raise RuntimeError(

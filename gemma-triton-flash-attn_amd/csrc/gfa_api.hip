@@ -222,6 +222,19 @@ int check_segments(const int32_t* lo, const int32_t* hi) {
   return GFA_OK;
 }
 
+// Arguments of the segment-table builders: `in` of elem-byte entries. The grid is one workgroup per
+// 1024 tokens and row.
+int check_table_args(const char* name, const void* in, int elem, int64_t row_stride, int B, int N, const int32_t* lo,
+                     const int32_t* hi) {
+  if (B <= 0 || N <= 0) return fail(GFA_ERR_INVALID_ARGUMENT, "empty table: batch=%d seq_len=%d", B, N);
+  if (B > 65535) return fail(GFA_ERR_UNSUPPORTED, "batch=%d rows exceed one launch grid", B);
+  if (in == nullptr || (reinterpret_cast<uintptr_t>(in) & (uintptr_t)(elem - 1)))
+    return fail(GFA_ERR_INVALID_ARGUMENT, "%s must be a pointer aligned to its %d-byte entries", name, elem);
+  if (row_stride < 0) return fail(GFA_ERR_INVALID_ARGUMENT, "%s has a negative row stride", name);
+  if (lo == nullptr || hi == nullptr) return fail(GFA_ERR_INVALID_ARGUMENT, "seg_lo and seg_hi are required");
+  return check_segments(lo, hi);
+}
+
 int check_dims(int B, int Hq, int Hkv, int N, int D, int dtype, int window) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || N <= 0)
     return fail(GFA_ERR_INVALID_ARGUMENT, "empty problem: B=%d Hq=%d Hkv=%d N=%d", B, Hq, Hkv, N);
@@ -756,6 +769,29 @@ int gfa_bwd_noalloc(const gfa_bwd_args* a) {
   if ((rc = scratch_on(static_cast<hipStream_t>(a->stream), &base))) return rc;
   char* p = static_cast<char*>(base);
   return bwd_impl(a, reinterpret_cast<float*>(p), ws ? p + delta_bytes : nullptr, ws, qs, false);
+}
+
+int gfa_segments_from_positions(const void* pos, int32_t pos_bits, int64_t row_stride, int32_t batch, int32_t seq_len,
+                                int32_t* seg_lo, int32_t* seg_hi, void* stream) {
+  if (pos_bits != 32 && pos_bits != 64) return fail(GFA_ERR_INVALID_ARGUMENT, "pos_bits=%d must be 32 or 64", pos_bits);
+  int rc = check_table_args("pos", pos, pos_bits / 8, row_stride, batch, seq_len, seg_lo, seg_hi);
+  if (rc) return rc;
+  const hipError_t err = gfa::launch_seg_positions(pos, pos_bits == 64, row_stride, batch, seq_len, seg_lo, seg_hi,
+                                                   static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(GFA_ERR_LAUNCH, "segment table launch failed: %s", hipGetErrorString(err));
+  return ok();
+}
+
+int gfa_segments_from_mask(const uint8_t* mask, int64_t row_stride, int32_t batch, int32_t seq_len, int32_t* seg_lo,
+                           int32_t* seg_hi, int32_t* bad, void* stream) {
+  int rc = check_table_args("mask", mask, 1, row_stride, batch, seq_len, seg_lo, seg_hi);
+  if (rc) return rc;
+  if (bad == nullptr || (reinterpret_cast<uintptr_t>(bad) & 3u))
+    return fail(GFA_ERR_INVALID_ARGUMENT, "bad must be a 4-byte aligned pointer");
+  const hipError_t err = gfa::launch_seg_mask(mask, row_stride, batch, seq_len, seg_lo, seg_hi, bad,
+                                              static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(GFA_ERR_LAUNCH, "segment table launch failed: %s", hipGetErrorString(err));
+  return ok();
 }
 
 }  // extern "C"

@@ -17,7 +17,8 @@ batches into tables:
   * ``from_cu_seqlens``    packed sequences: cumulative lengths over one row of N tokens;
   * ``from_position_ids``  packed sequences marked by position ids that restart.
 
-All run on the input's device with tensor operations; ``from_padding_mask`` and
+All run on the input's device, with tensor operations or, for masks and position ids on a GPU, in
+one kernel of the library (gfa_segments.hip); ``from_padding_mask`` and
 ``from_cu_seqlens`` check their input and raise ``ValueError`` for shapes a table cannot
 express (a padding mask whose real tokens are not one contiguous run). Those checks read
 device values on the host; under ``torch.compile`` (which cannot trace such reads) they are
@@ -30,6 +31,8 @@ as well-formed. A plain (lo, hi) tuple from elsewhere is checked there first
 from __future__ import annotations
 
 import torch
+
+from . import _lib
 
 
 class SegmentTables(tuple):
@@ -47,6 +50,58 @@ def _host_checks() -> bool:
     """Whether checks that read device values on the host may run (not while torch.compile
     traces: a data-dependent read would break its graph)."""
     return not torch.compiler.is_compiling()
+
+
+def _native(t: torch.Tensor) -> bool:
+    """Whether a table is built from ``t`` by the library's kernel (one launch): an ordinary tensor
+    on a GPU, outside tracing, function transforms and dispatch modes (which the tensor
+    operations below go through)."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.dim() == 2 and t.numel() > 0 and t.shape[0] <= 65535
+            and _host_checks() and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """``t`` with unit-stride rows (a batch expanded from one row stays a view)."""
+    return t if t.stride(1) == 1 and t.stride(0) >= 0 else t.contiguous()
+
+
+def _new_tables(t: torch.Tensor):
+    buf = torch.empty((2, *t.shape), dtype=torch.int32, device=t.device)
+    return buf[0], buf[1]
+
+
+class _RunCheck:
+    """The pending check of a padding mask whose tables a kernel is building: that kernel writes one
+    flag per row into pinned host memory, read once it has run (``done``, an event recorded
+    behind it). Calling it raises ValueError for a row whose real tokens are not one run. It must
+    be called (it also keeps the pinned memory until the kernel has written it)."""
+
+    def __init__(self, bad: torch.Tensor, done: torch.cuda.Event):
+        self.bad, self.done = bad, done
+
+    def __call__(self) -> None:
+        self.done.synchronize()
+        if any(self.bad.tolist()):
+            raise ValueError("padding mask rows must hold one contiguous run of real tokens (left or right padding)")
+
+
+def padding_tables(mask: torch.Tensor):
+    """``from_padding_mask`` without waiting for the check of the mask: (tables, check), where check()
+    raises ValueError for a mask a table cannot express, or is None (already checked). A caller
+    can launch the attention in between: the tables of a refused mask are in bounds."""
+    if not _native(mask):
+        return from_padding_mask(mask), None
+    m = _rows(mask if mask.dtype == torch.bool else mask.to(torch.bool))
+    lo, hi = _new_tables(m)
+    bad = torch.empty((m.shape[0],), dtype=torch.int32, pin_memory=True)
+    with torch.cuda.device(m.device):
+        stream = torch.cuda.current_stream()
+        _lib.check(_lib.load().gfa_segments_from_mask(m.data_ptr(), m.stride(0), m.shape[0], m.shape[1], lo.data_ptr(),
+                                                      hi.data_ptr(), bad.data_ptr(), stream.cuda_stream))
+        done = torch.cuda.Event()
+        done.record(stream)
+    return SegmentTables(lo, hi), _RunCheck(bad, done)
 
 
 def validate(lo: torch.Tensor, hi: torch.Tensor) -> None:
@@ -83,6 +138,10 @@ def from_padding_mask(mask: torch.Tensor) -> Segments:
     empty segments."""
     if mask.dim() != 2:
         raise ValueError(f"padding mask must be (B, N), got {tuple(mask.shape)}")
+    if _native(mask):
+        tables, check = padding_tables(mask)
+        check()
+        return tables
     m = mask.to(torch.bool)
     B, N = m.shape
     idx = torch.arange(N, device=m.device)
@@ -133,6 +192,14 @@ def from_position_ids(position_ids: torch.Tensor) -> Segments:
     """Packed sequences marked by position ids (B, N): a new sequence starts wherever the
     position id is not the previous one plus one (the rule transformers uses to detect
     packed batches, masking_utils.find_packed_sequence_indices)."""
+    if position_ids.dtype in (torch.int64, torch.int32) and _native(position_ids):
+        pos = _rows(position_ids)
+        lo, hi = _new_tables(pos)
+        with torch.cuda.device(pos.device):
+            _lib.check(_lib.load().gfa_segments_from_positions(
+                pos.data_ptr(), 8 * pos.element_size(), pos.stride(0), pos.shape[0], pos.shape[1], lo.data_ptr(),
+                hi.data_ptr(), torch.cuda.current_stream().cuda_stream))
+        return SegmentTables(lo, hi)
     pos = position_ids.to(torch.long)
     if pos.dim() == 1:
         pos = pos[None]

@@ -48,7 +48,7 @@
 extern "C" {
 #endif
 
-#define GFA_VERSION 106 /* 1.0.6: materialised backward (1.0.5: run-time work distribution, 1.0.4: attention dropout, 1.0.3: soft-capping) */
+#define GFA_VERSION 107 /* 1.0.7: segment tables from position ids and masks (1.0.6: materialised backward, 1.0.5: run-time work distribution, 1.0.4: attention dropout, 1.0.3: soft-capping) */
 
 typedef enum {
   GFA_DTYPE_FP16 = 0,
@@ -229,6 +229,21 @@ int gfa_config(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seq_len
  * results are bit for bit the same either way. enable = 0 launches the static grids; a negative
  * value only queries. Process-wide; returns the setting before the call. */
 int gfa_set_runtime_scheduling(int32_t enable);
+
+/* Segment tables built on the device (no counterpart in the reference), each one launch on `stream`
+ * that writes seg_lo and seg_hi, int32 (batch, seq_len) contiguous:
+ * - from position ids, int32 or int64 (pos_bits 32 or 64), row b at pos + b * row_stride elements (0:
+ *   one row for the whole batch): a sequence starts at token 0 and wherever the id is not the
+ *   previous one plus one;
+ * - from a padding mask, one byte per token (nonzero: a real token), row b at mask + b * row_stride:
+ *   the row's real tokens are one segment. bad (int32, batch entries, device or host-mapped
+ *   memory) receives 1 for a row whose real tokens are not one contiguous run, else 0; the table
+ *   of such a row is not a partition.
+ * seg_lo, seg_hi and bad must be 4-byte aligned, pos aligned to its type. Return a gfa_status. */
+int gfa_segments_from_positions(const void* pos, int32_t pos_bits, int64_t row_stride, int32_t batch, int32_t seq_len,
+                                int32_t* seg_lo, int32_t* seg_hi, void* stream);
+int gfa_segments_from_mask(const uint8_t* mask, int64_t row_stride, int32_t batch, int32_t seq_len, int32_t* seg_lo,
+                           int32_t* seg_hi, int32_t* bad, void* stream);
 
 /* Message of the last failing call on this thread ("" if none). */
 const char* gfa_last_error(void);

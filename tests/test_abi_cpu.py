@@ -310,3 +310,25 @@ def test_bwd_noalloc_rejects_caller_scratch_and_oversize():
     a.q_splits = 8
     assert lib.gfa_bwd_noalloc(ctypes.byref(a)) == 3
     assert lib.gfa_bwd_noalloc(None) == 1
+
+
+@fake_pointers
+def test_segment_table_builders_refuse_bad_arguments():
+    """Refused on the host, before any launch."""
+    lib = _lib.load()
+    pos = dict(pos=1024, bits=64, stride=8, B=1, N=8, lo=1024, hi=1024)
+
+    def positions(**kw):
+        a = {**pos, **kw}
+        return lib.gfa_segments_from_positions(a["pos"], a["bits"], a["stride"], a["B"], a["N"], a["lo"], a["hi"], None)
+
+    for kw in (dict(pos=None), dict(pos=1028), dict(bits=16), dict(stride=-1), dict(B=0), dict(N=0), dict(lo=None),
+               dict(hi=1026)):
+        assert positions(**kw) == 1, kw
+    assert positions(B=65536) == 2
+
+    def mask(m=1024, stride=8, B=1, N=8, lo=1024, hi=1024, bad=1024):
+        return lib.gfa_segments_from_mask(m, stride, B, N, lo, hi, bad, None)
+
+    for kw in (dict(m=None), dict(stride=-1), dict(B=0), dict(lo=None), dict(hi=1026), dict(bad=None), dict(bad=1026)):
+        assert mask(**kw) == 1, kw

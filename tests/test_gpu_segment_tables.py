@@ -1,0 +1,95 @@
+"""Segment tables built by the library's kernels (gfa_segments.hip) against the tensor operations of
+segments.py on the CPU (equal, whole numbers), at the edges of their 1024-token workgroups."""
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 2, 63, 64, 65, 1023, 1024, 1025, 2049, 5000]
+
+
+def _positions(kind, B, N):
+    g = torch.Generator().manual_seed(N)
+    pos = torch.arange(N).repeat(B, 1)
+    if kind == "packed":
+        for b in range(B):
+            cuts = [0] + sorted(int(x) for x in torch.randint(1, max(N, 2), (7,), generator=g)) + [N]
+            for a, e in zip(cuts, cuts[1:]):
+                pos[b, a:e] = torch.arange(max(0, e - a))
+    elif kind == "each":  # every token restarts
+        pos.zero_()
+    elif kind == "offset":  # one run that does not start at 0, and a restart at the last token
+        pos += 17
+        pos[-1, -1] = 3
+    return pos
+
+
+@pytest.mark.parametrize("N", SIZES)
+@pytest.mark.parametrize("kind", ["plain", "packed", "each", "offset"])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_positions(kind, N, dtype, device):
+    import gemma_triton_flash_attn_amd as gfa
+
+    pos = _positions(kind, 3, N).to(dtype)
+    want = gfa.segments.from_position_ids(pos)
+    wide = torch.zeros(3, N + 5, dtype=dtype, device=device)
+    wide[:, :N] = pos.to(device)
+    for p in (pos.to(device), wide[:, :N]):
+        got = gfa.segments.from_position_ids(p)
+        assert isinstance(got, gfa.segments.SegmentTables)
+        assert all(torch.equal(a.cpu(), b) and a.dtype == torch.int32 for a, b in zip(got, want))
+    row = gfa.segments.from_position_ids(pos[:1].to(device).expand(4, N))  # one row for the batch
+    assert all(torch.equal(a.cpu(), b[:1].expand(4, N)) for a, b in zip(row, want))
+
+
+@pytest.mark.parametrize("N", SIZES)
+@pytest.mark.parametrize("dtype", [torch.bool, torch.int64])
+def test_masks(N, dtype, device):
+    import gemma_triton_flash_attn_amd as gfa
+
+    i = torch.arange(N)
+    rows = [i < N, i < (N + 1) // 2, i >= N // 3, (i >= N // 4) & (i < 1 + N // 2), i < 0, i == N - 1]
+    mask = torch.stack(rows).to(dtype)
+    want = gfa.segments.from_padding_mask(mask)
+    got = gfa.segments.from_padding_mask(mask.to(device))
+    assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
+    if N >= 3:
+        holed = mask.clone()
+        holed[0, N // 2] = 0
+        for m in (holed, holed[:1]):
+            with pytest.raises(ValueError, match="contiguous"):
+                gfa.segments.from_padding_mask(m.to(device))
+
+
+@pytest.mark.parametrize("N", [70, 1500])
+def test_adapter(N, device):
+    """The adapter with position ids and masks: the same output as with tables built by hand, and a
+    mask with holes still refused."""
+    import gemma_triton_flash_attn_amd as gfa
+
+    g = torch.Generator().manual_seed(N)
+    q = torch.randn(2, N, 4, 256, generator=g).to(device, torch.bfloat16).transpose(1, 2)
+    k, v = (torch.randn(2, N, 2, 256, generator=g).to(device, torch.bfloat16).transpose(1, 2) for _ in range(2))
+    mod = SimpleNamespace(head_dim=256, is_causal=True)
+
+    def want(segs):
+        return gfa.attention_flash_gqa(q, k, v, causal=True, segments=segs).transpose(1, 2)
+
+    plain, _ = gfa.triton_gqa_attention(mod, q, k, v, None, position_ids=torch.arange(N, device=device)[None])
+    assert torch.equal(plain, want(None))
+    pos = _positions("packed", 2, N)
+    packed, _ = gfa.triton_gqa_attention(mod, q, k, v, None, position_ids=pos.to(device))
+    assert torch.equal(packed, want(tuple(t.to(device) for t in gfa.segments.from_position_ids(pos))))
+    mask = torch.arange(N)[None] < torch.tensor([[N], [N // 2]])
+    padded, _ = gfa.triton_gqa_attention(mod, q, k, v, mask.to(device))
+    assert torch.equal(padded, want(tuple(t.to(device) for t in gfa.segments.from_padding_mask(mask))))
+    mask[1, 3] = False
+    with pytest.raises(NotImplementedError, match="contiguous"):
+        gfa.triton_gqa_attention(mod, q, k, v, mask.to(device))
+    # three rows of ids for two rows of tokens: unpacked ids describe no segments, as before
+    odd, _ = gfa.triton_gqa_attention(mod, q, k, v, None, position_ids=torch.arange(N, device=device).repeat(3, 1))
+    assert torch.equal(odd, plain)
