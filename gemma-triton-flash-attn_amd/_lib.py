@@ -9,6 +9,8 @@ raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -16,6 +18,7 @@ import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("GFA_LIBRARY", os.path.join(_HERE, "libgfa.so"))
+TORCH_LIB_PATH = os.path.join(_HERE, "_gfa_torch.so")
 
 GFA_DTYPE_FP16 = 0
 GFA_DTYPE_BF16 = 1
@@ -144,6 +147,37 @@ def load() -> ctypes.CDLL:
                 "rebuild it with `python gemma-triton-flash-attn_amd/build.py` (or __graft_entry__.build())")
         _lib = lib
         return lib
+
+
+_native = None
+
+
+def native():
+    """The C++ host path (_gfa_torch.so, csrc/gfa_torch.cpp), loaded once and bound to the C ABI of
+    load()'s library. Raises if it is missing or was built for another version."""
+    global _native
+    if _native is not None:
+        return _native
+    lib = load()
+    with _lock:
+        if _native is not None:
+            return _native
+        rebuild = "rebuild with `python gemma-triton-flash-attn_amd/build.py` (or __graft_entry__.build())"
+        if not os.path.exists(TORCH_LIB_PATH):
+            raise RuntimeError(f"{TORCH_LIB_PATH} not found; {rebuild}")
+        loader = importlib.machinery.ExtensionFileLoader("_gfa_torch", TORCH_LIB_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_gfa_torch", loader))
+        loader.exec_module(mod)
+        if mod.version != ABI_VERSION:
+            raise RuntimeError(f"{TORCH_LIB_PATH} was built for GFA_VERSION {mod.version}, not {ABI_VERSION}; {rebuild}")
+
+        def address(name):
+            return ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+
+        mod.bind(address("gfa_fwd"), address("gfa_bwd"), address("gfa_bwd_workspace_bytes"),
+                 address("gfa_segments_from_positions"), address("gfa_last_error"), GfaError)
+        _native = mod
+        return mod
 
 
 def check(status: int) -> None:

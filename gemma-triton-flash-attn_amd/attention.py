@@ -314,6 +314,35 @@ class FlashAttnGQAFunction(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None, None, None
 
 
+def _native_call(q, k, v) -> bool:
+    """Whether a call takes the C++ host path (_lib.native(): the same launches, allocations and
+    autograd formula as below, without the interpreter): ordinary tensors, outside compilation,
+    tracing, function transforms and dispatch modes, which see the Python autograd function or the
+    registered op as before."""
+    return (type(q) in _ORDINARY and type(k) in _ORDINARY and type(v) in _ORDINARY
+            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._functorch.peek_interpreter_stack() is None)
+
+
+_ORDINARY = (torch.Tensor, torch.nn.Parameter)
+
+
+def _attend(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p, grad: bool):
+    """The C++ host path after the checks of FlashAttnGQAFunction.forward; ``grad``: with autograd."""
+    _check_inputs(q, k, v)
+    segments = _check_segments(segments, q)
+    window = _norm_window(causal, slide_size, q.shape[2])
+    sc = _default_scale(q.shape[3], scale)
+    cap = _check_softcap(softcap)
+    dp = _check_dropout(dropout_p)
+    _check_cap_and_dropout(cap, dp)
+    seed = _dropout_seed() if dp > 0.0 else 0
+    lo, hi = segments if segments is not None else (None, None)
+    if grad:
+        return _lib.native().train(q, k, v, bool(causal), window, sc, cap, dp, seed, lo, hi)
+    return _lib.native().infer(q, k, v, bool(causal), window, sc, cap, dp, seed, 0, lo, hi)
+
+
 def flash_attn_gqa_train(q, k, v, causal=False, slide_size=0, *, scale=None, segments=None, softcap=None,
                          dropout_p=0.0):
     """Flash attention with autograd support (reference attention.py:1625-1635).
@@ -326,6 +355,8 @@ def flash_attn_gqa_train(q, k, v, causal=False, slide_size=0, *, scale=None, seg
     ``dropout_p``: attention dropout on the softmax probabilities (kept ones scaled by
     1 / (1 - p)), with a fresh mask seed from torch's generator per call; not in the reference.
     """
+    if _native_call(q, k, v):
+        return _attend(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p, grad=True)
     return FlashAttnGQAFunction.apply(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p)
 
 
@@ -349,7 +380,12 @@ def attention_flash_gqa(q, k, v, causal=False, slide_size=0, BLOCK_Q=None, BLOCK
     if BLOCK_D is not None and int(BLOCK_D) != D:
         raise ValueError("BLOCK_D must equal HEAD_DIM (no head-dim tiling)")
     slide_size = _norm_window(causal, slide_size, q.shape[2])
-    o, _ = _forward(q, k, v, causal, slide_size, _default_scale(D, scale), store_lse=False, block_kv=bkv,
-                    segments=_check_segments(segments, q), softcap=_check_softcap(softcap))
+    scale = _default_scale(D, scale)
+    segments = _check_segments(segments, q)
+    cap = _check_softcap(softcap)
+    if _native_call(q, k, v):
+        lo, hi = segments if segments is not None else (None, None)
+        return _lib.native().infer(q, k, v, bool(causal), slide_size, scale, cap, 0.0, 0, bkv, lo, hi)
+    o, _ = _forward(q, k, v, causal, slide_size, scale, store_lse=False, block_kv=bkv, segments=segments, softcap=cap)
     return o
 

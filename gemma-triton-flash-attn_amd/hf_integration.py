@@ -12,10 +12,11 @@ Differences from the reference adapter:
   * the output is allocated with q's strides, so for transformers' transposed
     (B, H, N, D) views of (B, N, H, D) projections the final ``transpose(1, 2)`` is
     already contiguous and ``.contiguous()`` does not copy (reference 75);
-  * the call goes through the registered ``gfa::attn_fwd`` op (``ops.py``), so a model
-    under ``torch.compile`` keeps one graph across its attention layers. The op launches on
-    its tensors' device itself, which replaces the reference's ``torch.cuda.device`` guard
-    (68-74);
+  * under ``torch.compile`` (and any other tracing or dispatch mode) the call goes through the
+    registered ``gfa::attn_fwd`` op (``ops.py``), so a model keeps one graph across its
+    attention layers; an eager call takes the C++ host path (``attention._native_call``), the
+    same launches at a third of the host time. Both launch on their tensors' device
+    themselves, which replaces the reference's ``torch.cuda.device`` guard (68-74);
   * padded and packed batches are computed, not ignored (the reference adapter drops
     ``attention_mask``, 43-47): a padding mask, ``cu_seq_lens_*`` or restarting
     ``position_ids`` become segment tables (segments.py) for the kernels.
@@ -25,6 +26,7 @@ from __future__ import annotations
 import torch
 
 from . import segments as seglib
+from .attention import _attend, _native_call
 from .ops import flash_attn_gqa_op
 
 
@@ -99,8 +101,13 @@ def triton_gqa_attention(module, query, key, value, attention_mask, dropout: flo
         scale = scaling if scaling is not None else module.head_dim ** -0.5
         slide = int(sliding_window) if sliding_window else 0
         is_causal = getattr(module, "is_causal", True)
-        out = flash_attn_gqa_op(query, key, value, causal=is_causal, slide_size=slide, scale=scale, segments=segments,
-                                softcap=softcap, dropout_p=float(dropout or 0.0))
+        drop = float(dropout or 0.0)
+        if _native_call(query, key, value):
+            grad = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
+            out = _attend(query, key, value, is_causal, slide, scale, segments, softcap, drop, grad)
+        else:
+            out = flash_attn_gqa_op(query, key, value, causal=is_causal, slide_size=slide, scale=scale,
+                                    segments=segments, softcap=softcap, dropout_p=drop)
     finally:
         for check in checks:
             try:

@@ -193,13 +193,7 @@ def from_position_ids(position_ids: torch.Tensor) -> Segments:
     position id is not the previous one plus one (the rule transformers uses to detect
     packed batches, masking_utils.find_packed_sequence_indices)."""
     if position_ids.dtype in (torch.int64, torch.int32) and _native(position_ids):
-        pos = _rows(position_ids)
-        lo, hi = _new_tables(pos)
-        with torch.cuda.device(pos.device):
-            _lib.check(_lib.load().gfa_segments_from_positions(
-                pos.data_ptr(), 8 * pos.element_size(), pos.stride(0), pos.shape[0], pos.shape[1], lo.data_ptr(),
-                hi.data_ptr(), torch.cuda.current_stream().cuda_stream))
-        return SegmentTables(lo, hi)
+        return SegmentTables(*_lib.native().positions(_rows(position_ids)))
     pos = position_ids.to(torch.long)
     if pos.dim() == 1:
         pos = pos[None]
