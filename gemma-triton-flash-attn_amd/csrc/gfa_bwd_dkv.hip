@@ -8,8 +8,8 @@
 // with P and dS recomputed from LSE and delta exactly as in the dQ kernel, P and dS cast
 // to the input dtype before the products. The query range of a key block starts at the
 // key block (causal) and ends at the last key + window - 1 (sliding window).
-// With q_splits > 1 the (head, query tile) iteration space of every key block is cut into
-// q_splits contiguous chunks; each chunk writes an fp32 partial (scaled) and
+// With q_splits > 1 the (head, query tile) iteration space of a key block is cut into up to
+// q_splits contiguous chunks (dkv_splits); each chunk writes an fp32 partial (scaled) and
 // dkv_reduce_kernel sums them in a fixed order (deterministic, no atomics; the reference
 // uses atomic_add into 16-bit dK/dV, attention.py:1206-1209).
 //
@@ -55,36 +55,34 @@ constexpr bool dkv_stages_rows(int D, int roles) { return roles == 1 && D >= 128
 #undef GFA_DKV_KERNEL
 #undef GFA_DKV_STORE
 
-// dK/dV = sum over q_splits of the fp32 partials, in split order, cast to the input dtype.
-// One thread converts 8 consecutive head-dim elements of one (tensor, b, kvh, key) row.
+// dK/dV = sum over a key block's splits of the fp32 partials, in split order, cast to the input
+// dtype; blocks with one split are written by their workgroup. One thread converts 8 consecutive
+// head-dim elements of one row; blockIdx.y is the (tensor, b, kvh) plane.
 template <bool IS_BF16>
-__global__ __launch_bounds__(256) void dkv_reduce_kernel(const BwdDkvParams p, int D) {
-  const int64_t plane = (int64_t)p.B * p.Hkv * p.N * D;
-  const int64_t n8 = 2 * plane / 8;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n8) return;
-  const int64_t e0 = i * 8;
-  const int which = e0 >= plane ? 1 : 0;
-  const int64_t off = e0 - which * plane;
+__global__ __launch_bounds__(256) void dkv_reduce_kernel(const BwdDkvParams p, int log2_d) {
+  const int64_t rows = (int64_t)p.B * p.Hkv * p.N << log2_d;  // elements of one tensor
+  const int64_t off = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  const int key = (int)(off >> log2_d);
+  if (key >= p.N) return;
+  const int splits = p.chunk == 0 ? p.q_splits : dkv_splits(p, key / p.wkv * p.wkv);
+  if (splits == 1) return;
+  const int planes = p.B * p.Hkv;
+  const int which = blockIdx.y >= planes;
+  const int bk = blockIdx.y - which * planes;
+  const float* src = p.part + which * rows + ((int64_t)bk * p.N << log2_d) + off;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int s = 0; s < p.q_splits; ++s) {
-    const float* src = p.part + (int64_t)s * 2 * plane + which * plane + off;
-    const f32x4 a = *reinterpret_cast<const f32x4*>(src);
-    const f32x4 c = *reinterpret_cast<const f32x4*>(src + 4);
+  for (int s = 0; s < splits; ++s) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(src + s * 2 * rows);
+    const f32x4 c = *reinterpret_cast<const f32x4*>(src + s * 2 * rows + 4);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       acc[e] += a[e];
       acc[4 + e] += c[e];
     }
   }
-  const int d = (int)(off % D);
-  int64_t rest = off / D;
-  const int key = (int)(rest % p.N);
-  rest /= p.N;
-  const int kvh = (int)(rest % p.Hkv);
-  const int b = (int)(rest / p.Hkv);
   const RowView& v = which ? p.dvv : p.dkv;
-  uint16_t* dst = (which ? p.dv : p.dk) + (int64_t)b * v.sb + (int64_t)kvh * v.sh + (int64_t)key * v.sn + d;
+  uint16_t* dst = (which ? p.dv : p.dk) + (int64_t)(bk / p.Hkv) * v.sb + (int64_t)(bk % p.Hkv) * v.sh +
+                  (int64_t)key * v.sn + (off & ((1 << log2_d) - 1));
   i16x8 o;
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = to16<IS_BF16>(acc[e]);
@@ -92,9 +90,11 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const BwdDkvParams p, i
 }
 
 // Explicit instantiations of every built variant (device code and host launch stubs).
-#define GFA_DKV_INST(DD, BB, WW, RR, EE, CC, XX)                                                  \
-  template __global__ void bwd_dkv_kernel<DD, BB, true, WW, RR, EE, CC, XX>(const BwdDkvParams);  \
-  template __global__ void bwd_dkv_kernel<DD, BB, false, WW, RR, EE, CC, XX>(const BwdDkvParams);
+#define GFA_DKV_INST(DD, BB, WW, RR, EE, CC, XX)                                                         \
+  template __global__ void bwd_dkv_kernel<DD, BB, true, WW, RR, EE, CC, XX, false>(const BwdDkvParams);  \
+  template __global__ void bwd_dkv_kernel<DD, BB, false, WW, RR, EE, CC, XX, false>(const BwdDkvParams); \
+  template __global__ void bwd_dkv_kernel<DD, BB, true, WW, RR, EE, CC, XX, true>(const BwdDkvParams);   \
+  template __global__ void bwd_dkv_kernel<DD, BB, false, WW, RR, EE, CC, XX, true>(const BwdDkvParams);
 GFA_DKV_INST(512, 32, 4, 2, 1, false, false)
 GFA_DKV_INST(256, 32, 4, 1, 1, false, false)
 GFA_DKV_INST(256, 32, 4, 2, 2, false, false)
@@ -111,9 +111,11 @@ GFA_DKV_EXT(true, false)
 GFA_DKV_EXT(false, true)
 #undef GFA_DKV_EXT
 #undef GFA_DKV_INST
-#define GFA_DKV_DS_INST(CC, XX)                                                                     \
-  template __global__ void bwd_dkv_ds_kernel<256, 32, true, 4, 1, 1, CC, XX>(const BwdDkvParams);  \
-  template __global__ void bwd_dkv_ds_kernel<256, 32, false, 4, 1, 1, CC, XX>(const BwdDkvParams);
+#define GFA_DKV_DS_INST(CC, XX)                                                                            \
+  template __global__ void bwd_dkv_ds_kernel<256, 32, true, 4, 1, 1, CC, XX, false>(const BwdDkvParams);  \
+  template __global__ void bwd_dkv_ds_kernel<256, 32, false, 4, 1, 1, CC, XX, false>(const BwdDkvParams); \
+  template __global__ void bwd_dkv_ds_kernel<256, 32, true, 4, 1, 1, CC, XX, true>(const BwdDkvParams);   \
+  template __global__ void bwd_dkv_ds_kernel<256, 32, false, 4, 1, 1, CC, XX, true>(const BwdDkvParams);
 GFA_DKV_DS_INST(false, false)
 GFA_DKV_DS_INST(true, false)
 GFA_DKV_DS_INST(false, true)
@@ -121,19 +123,28 @@ GFA_DKV_DS_INST(false, true)
 template __global__ void dkv_reduce_kernel<true>(const BwdDkvParams, int);
 template __global__ void dkv_reduce_kernel<false>(const BwdDkvParams, int);
 
-template <int D, int BQ, bool IS_BF16, int NW, int ROLES, int WPE, bool CAP, bool DROP>
-static hipError_t launch_dkv_t(const BwdDkvParams& p, hipStream_t stream) {
+template <int D, int BQ, bool IS_BF16, int NW, int ROLES, int WPE, bool CAP, bool DROP, bool CHUNKED>
+static hipError_t launch_dkv_c(const BwdDkvParams& p, hipStream_t stream) {
   const unsigned stage_bytes = dkv_stages_rows(D, ROLES) ? NW * BQ * D * 2 : 0;  // the kernel's stage_raw
   if constexpr (ROLES == 1 && D == 256) {
     if (p.dsl.ds != nullptr) {
-      hipLaunchKernelGGL((bwd_dkv_ds_kernel<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP>), dim3(p.nblocks),
+      hipLaunchKernelGGL((bwd_dkv_ds_kernel<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP, CHUNKED>), dim3(p.nblocks),
                          dim3(NW * 64), stage_bytes, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((bwd_dkv_kernel<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP>), dim3(p.nblocks), dim3(NW * 64),
-                     stage_bytes, stream, p);
+  hipLaunchKernelGGL((bwd_dkv_kernel<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP, CHUNKED>), dim3(p.nblocks),
+                     dim3(NW * 64), stage_bytes, stream, p);
   return hipGetLastError();
+}
+
+// Grids with a split count per key block (p.chunk > 0) run instances of their own: with their block
+// search in it, the kernel of the other grids is 0.7% slower at the headline and 1.3% on the
+// window-512 layer.
+template <int D, int BQ, bool IS_BF16, int NW, int ROLES, int WPE, bool CAP, bool DROP>
+static hipError_t launch_dkv_t(const BwdDkvParams& p, hipStream_t stream) {
+  return p.chunk > 0 ? launch_dkv_c<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP, true>(p, stream)
+                     : launch_dkv_c<D, BQ, IS_BF16, NW, ROLES, WPE, CAP, DROP, false>(p, stream);
 }
 
 // Built dK/dV variants: (head dim, queries per tile, waves per workgroup, waves per 32 keys,
@@ -162,13 +173,14 @@ hipError_t launch_bwd_dkv(const BwdDkvParams& p, int D, int bq, int nw, int role
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_dkv_reduce(const BwdDkvParams& p, int D, bool bf16, hipStream_t stream) {
-  const int64_t n8 = 2 * (int64_t)p.B * p.Hkv * p.N * D / 8;
-  const int blocks = (int)((n8 + 255) / 256);
+hipError_t launch_dkv_reduce(const BwdDkvParams& p, int head_dim, bool bf16, hipStream_t stream) {
+  const int log2_d = head_dim == 512 ? 9 : head_dim == 256 ? 8 : head_dim == 128 ? 7 : 6;
+  const int64_t per_plane = ((int64_t)p.N << log2_d) / 8;
+  const dim3 grid((unsigned)((per_plane + 255) / 256), 2 * p.B * p.Hkv);
   if (bf16) {
-    hipLaunchKernelGGL(dkv_reduce_kernel<true>, dim3(blocks), dim3(256), 0, stream, p, D);
+    hipLaunchKernelGGL(dkv_reduce_kernel<true>, grid, dim3(256), 0, stream, p, log2_d);
   } else {
-    hipLaunchKernelGGL(dkv_reduce_kernel<false>, dim3(blocks), dim3(256), 0, stream, p, D);
+    hipLaunchKernelGGL(dkv_reduce_kernel<false>, grid, dim3(256), 0, stream, p, log2_d);
   }
   return hipGetLastError();
 }

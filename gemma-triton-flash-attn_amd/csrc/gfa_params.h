@@ -118,12 +118,36 @@ struct BwdDkvParams {
   float inv_scale;   // 1 / scale
   SoftCap cap;       // read by the CAP instances only
   Dropout drop;      // read by the DROP instances only
-  int q_splits;
+  int q_splits;      // most splits of a key block's query range (planes of `part`)
+  int chunk;         // > 0: a block's splits are its iterations over this (dkv_splits); 0: q_splits each
   int lse_ld;
   int n_kb;          // number of key blocks (each WKV keys wide)
-  int nblocks;       // q_splits * B * Hkv * n_kb rounded up to whole groups of four key blocks
+  int wkv;           // keys per key block
+  int nblocks;       // workgroups: B * Hkv * n_kb in whole groups of four key blocks, or the splits' sum
   DsLayout dsl;      // dS store (dsl.ds null: none)
 };
+
+// Iterations (query tiles x heads, before any segment table trims them) of the key block that starts
+// at key k0.
+__host__ __device__ inline int dkv_iterations(const BwdDkvParams& p, int k0) {
+  int end = (p.N + 31) / 32;
+  if (p.causal && p.window > 0) {
+    const int last = (k0 + p.wkv < p.N ? k0 + p.wkv : p.N) - 1;
+    const int e = (last + p.window - 1) / 32 + 1;
+    if (e < end) end = e;
+  }
+  return p.R * (end - (p.causal ? k0 / 32 : 0));
+}
+// Its splits: q_splits with chunk == 0, else its iterations over `chunk`, at most q_splits. A block
+// with one split writes its rows directly; the reduction sums the planes of the others.
+__host__ __device__ inline int dkv_splits_of(int iterations, int chunk, int q_splits) {
+  if (chunk == 0) return q_splits;
+  const int n = (iterations + chunk - 1) / chunk;
+  return n < 1 ? 1 : n < q_splits ? n : q_splits;
+}
+__host__ __device__ inline int dkv_splits(const BwdDkvParams& p, int k0) {
+  return dkv_splits_of(dkv_iterations(p, k0), p.chunk, p.q_splits);
+}
 
 // delta = rowsum(dO * O) of every row of the 32-row tiles that cover N (rows past N repeat row
 // N - 1), for the materialised backward, whose dQ kernel no longer computes it.

@@ -121,7 +121,8 @@ typedef struct {
   int32_t causal, window;
   float scale;
   int32_t dtype;
-  int32_t q_splits;       /* 0 = registry choice, else 1, 2, 4 or 8 */
+  int32_t q_splits;       /* 0 = registry choice, else 1, 2, 4 or 8: the most splits of a key
+                             block's query range (blocks with a short range may get fewer) */
   int32_t lse_ld;         /* row length of lse and delta (>= GFA_LSE_LD(seq_len)) */
   int32_t stages;         /* 0 = all; else bitwise OR of GFA_BWD_DQ and GFA_BWD_DKV (profiling:
                              recomputing form: GFA_BWD_DKV alone reads the delta a previous
