@@ -148,6 +148,10 @@ gfa::QGrid make_qgrid(int B, int Hkv, int R, int N, int nu) {
 //   only from 1024 tokens (D=128 32:8 N=333 10.6 -> 11.8 us).
 // Past that the K / V copies per 32 rows cost more than the idle CUs (D=512 8:1 N=3000, 752
 // blocks: 128 -> 142 us; windows: D=256 8:1 W=512 N=1500, 376 blocks: 20.2 -> 23.5 us).
+// The dQ kernel of the materialised backward has the same two forms and the same line
+// (bwd_dq_rows_kernel against bwd_dq_ds_kernel): D=512 8:1 N=1024 31.6 -> 15.2 us, N=2000 57.2 -> 40.8,
+// 16:2 N=1300 (656 blocks) 42.8 -> 39.3, N=2048 (1024) 62.2 -> 75.0; D=256 8:4 N=2048 32.8 -> 24.2, N=3000
+// (752) 46.0 -> 49.0; window 512 8:1 N=800 (200) 13.6 -> 9.2, N=2000 (504) 14.3 -> 17.1.
 bool use_rows_kernel(int D, int B, int Hq, int N, bool causal, bool windowed) {
   const long long blocks = (long long)B * Hq * ((N + 31) / 32);
   if (D == 64 && N <= 128) return false;
@@ -749,8 +753,13 @@ int bwd_impl(const gfa_bwd_args* a, float* delta_buf, void* ws_buf, size_t ws_by
       pz.R = R;
       pz.scale = a->scale;
       pz.dsl = pk.dsl;
-      pz.g = make_qgrid(pz.B, pz.Hkv, R, pz.N, 4);
-      err = gfa::launch_bwd_dq_ds(pz, a->head_dim, bf16, stream);
+      if (use_rows_kernel(a->head_dim, pz.B, pz.Hq, pz.N, pq.causal, window > 0)) {
+        pz.g = rows_grid(pz.B, pz.Hkv, R, pz.N);
+        err = gfa::launch_bwd_dq_rows(pz, a->head_dim, bf16, stream);
+      } else {
+        pz.g = make_qgrid(pz.B, pz.Hkv, R, pz.N, 4);
+        err = gfa::launch_bwd_dq_ds(pz, a->head_dim, bf16, stream);
+      }
       if (err != hipSuccess) return fail(GFA_ERR_LAUNCH, "dQ (from dS) launch failed: %s", hipGetErrorString(err));
     }
     return ok();

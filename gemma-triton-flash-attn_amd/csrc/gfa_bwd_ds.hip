@@ -420,9 +420,212 @@ __global__ __launch_bounds__(256, WPE) void bwd_dq_ds_kernel(const BwdDqDsParams
   put(u0 + 1, stg1);
 }
 
+// dQ from the dS store for small grids: a workgroup owns one (head, 32-row query tile) unit and its
+// waves split the key tiles, as fwd_rows_kernel does. A wave (D = 256) or a wave pair (D = 512, each
+// wave over one half of the head dim) is a key group: it accumulates dQ^T over the tiles
+// jlo + g, jlo + g + NG, ... of the unit's row of blocks from private copies of the K tile and the
+// dS block, so the loop has no workgroup barrier, and the groups' sums are added through LDS in
+// fp32 at the end. bwd_dq_ds_kernel's four units per workgroup read a K tile once per 128 rows, but
+// leave CUs idle on a short sequence and walk its keys serially (D=512 8:1 N=1024: 64 workgroups, 31.6 us; 256 and 15.2 us here;
+// gfa_api.hip, use_rows_kernel). Bound: the K copies, 32 rows per tile byte.
+// K tiles are double buffered, copied two instructions per product behind the first half of the
+// products of the tile before; a dS block's slot is free once its operands are in registers and
+// takes the block two tiles ahead (the store is further away than a tile's time).
+template <int D, bool IS_BF16>
+__global__ __launch_bounds__(256, 1) void bwd_dq_rows_kernel(const BwdDqDsParams p) {
+  constexpr int SD = D / 256;  // waves per key group, each over DW columns
+  constexpr int NG = 4 / SD;
+  constexpr int DW = 256;
+  constexpr int DB = DW / 32;
+  constexpr int HALF = 16 * DW * 2;  // half a K tile: rows 0..15 or 16..31
+  constexpr int DSB = 2048;
+  // One LDS object per half tile and parity (the compiler waits for every copy into an object it
+  // reads): [parity][half], a block per wave.
+  __shared__ __attribute__((aligned(1024))) char k_lds00[4 * HALF], k_lds01[4 * HALF];
+  __shared__ __attribute__((aligned(1024))) char k_lds10[4 * HALF], k_lds11[4 * HALF];
+  __shared__ __attribute__((aligned(1024))) char s_lds0[4 * DSB];
+  __shared__ __attribute__((aligned(1024))) char s_lds1[4 * DSB];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave / SD;
+  const int dh = wave % SD;
+  const int h = lane >> 5;
+  char GFA_LDS* const K00 = (char GFA_LDS*)k_lds00 + wave * HALF;
+  char GFA_LDS* const K01 = (char GFA_LDS*)k_lds01 + wave * HALF;
+  char GFA_LDS* const K10 = (char GFA_LDS*)k_lds10 + wave * HALF;
+  char GFA_LDS* const K11 = (char GFA_LDS*)k_lds11 + wave * HALF;
+  char GFA_LDS* const S0 = (char GFA_LDS*)s_lds0 + wave * DSB;
+  char GFA_LDS* const S1 = (char GFA_LDS*)s_lds1 + wave * DSB;
+
+  int lid = xcd_remap((int)blockIdx.x, p.g.nblocks, p.g.n_hg);
+  const int hg = lid % p.g.n_hg;
+  lid /= p.g.n_hg;
+  const int kvh = lid % p.Hkv;
+  lid /= p.Hkv;
+  const int b = lid % p.B;
+  lid /= p.B;
+  const int qt = p.dsl.mode == 1 ? (p.g.n_qsb - 1 - lid) : lid;  // full causal: longest rows first
+  const int head = kvh * p.R + hg;
+
+  // The unit's blocks [jlo, jhi], and this group's share of them.
+  int jlo = ds_jmin(p.dsl, qt), jhi = ds_jmax(p.dsl, qt);
+  if (p.seg_lo) {
+    int a, c;
+    ds_seg_units(p.seg_lo + (int64_t)b * p.N, p.seg_hi + (int64_t)b * p.N, p.N, qt, &a, &c);
+    jlo = max(jlo, a);
+    jhi = min(jhi, c);
+  }
+  const int steps = max(0, (jhi - jlo - grp + NG) / NG);
+
+  TileLoader<DW, 32, 1> kload;
+  kload.init(p.k + (int64_t)b * p.kv.sb + (int64_t)kvh * p.kv.sh + dh * DW, p.kv.sn, p.N, 0, lane);
+  constexpr int NI = TileLoader<DW, 32, 1>::NI;
+  static_assert(NI == 16, "two copies behind each of the first eight products");
+  const uint16_t* row = p.dsl.ds + ((int64_t)b * p.Hq + head) * p.dsl.slab * 1024 +
+                        (jlo <= jhi ? ds_index(p.dsl, qt, jlo) * 1024 : 0);  // the unit's first block
+  unsigned svoff[2];  // as bwd_dq_ds_kernel: key row r of part c at r ^ 4c
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = 2 * i + h;
+    svoff[i] = (unsigned)(c * 512 + 16 * ((lane & 31) ^ (4 * c)));
+  }
+  // Block of step s (past the last one: an empty resource, zeros), and the first key of its tile
+  // (past the last one: the sequence end, zeros).
+  auto copy_ds = [&](int s, char GFA_LDS* buf) __attribute__((always_inline)) {
+    const bool have = s < steps;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(row + (have ? (int64_t)(grp + s * NG) * 1024 : 0)), 0, have ? DSB : 0, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void GFA_LDS*)(buf + c * 1024), 16, svoff[c], 0, 0, 2 /* nt */);
+  };
+  auto key_of = [&](int s) __attribute__((always_inline)) { return s < steps ? (jlo + grp + s * NG) * 32 : p.N; };
+
+  int toffA, toffB, soffA, soffB;  // column block 0: block db at ^ (db & 3) << 6, + 256 (db >> 2)
+  {
+    const int t16 = lane & 15;
+    const int rA = 4 * h + (t16 >> 2);
+    const int c = 2 * ((lane >> 4) & 1) + ((t16 >> 1) & 1);
+    toffA = rA * (2 * DW) + ((c ^ swz<DW>(rA)) << 4) + (t16 & 1) * 8;
+    toffB = (toffA ^ 32) + 16 * DW;  // 8 rows further down (mma_tr_accumulate_b)
+    soffA = c * 512 + 16 * (rA ^ (4 * c)) + (t16 & 1) * 8;
+    soffB = c * 512 + 16 * ((rA + 8) ^ (4 * c)) + (t16 & 1) * 8;
+  }
+
+  f32x16 acc[DB];
+#pragma unroll
+  for (int i = 0; i < DB; ++i) acc[i] = f32x16{};
+
+  // Copy instruction i (two rows) of the tile at key row0 into its halves ka, kb.
+  auto kcopy = [&](int i, int row0, char GFA_LDS* ka, char GFA_LDS* kb) __attribute__((always_inline)) {
+    kload.load_part(i, row0, i < NI / 2 ? ka : kb - HALF);  // (instruction i writes at 1 KB * i)
+  };
+  // Step s: its tile in ka, kb, its block in st; the next tile goes to na, nb, the block two steps
+  // ahead to st. Copies in issue order: block s, tile s - 1, block s + 1, tile s (rows 0..15, 16..31).
+  auto step = [&](int s, const char GFA_LDS* ka, const char GFA_LDS* kb, char GFA_LDS* st, char GFA_LDS* na,
+                  char GFA_LDS* nb) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // block s, rows 0..15 of tile s
+    i16x8 b[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) b[ks] = tr_frag(st, soffA, soffB, ks * 256);
+    constexpr int PF = 4;
+    auto frag = [&](int i) __attribute__((always_inline)) {
+      const int db = i % DB, x = (db & 3) << 6;
+      return tr_frag(i < DB ? ka : kb, toffA ^ x, toffB ^ x, 256 * (db >> 2));
+    };
+    i16x8 a[PF];
+#pragma unroll
+    for (int i = 0; i < PF; ++i) a[i] = frag(i);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the block's operands are in registers
+    copy_ds(s + 2, st);
+    const int next = key_of(s + 1);
+#pragma unroll
+    for (int i = 0; i < 2 * DB; ++i) {
+      const i16x8 cur = a[i % PF];
+      // rows 16..31, first read PF products ahead: two block copies and 2 (i + 1) - 2 of the next tile behind them
+      if (i + PF == DB) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + 2 * (DB - PF)) : "memory");
+      if (i + PF < 2 * DB) a[i % PF] = frag(i + PF);
+      acc[i % DB] = mma32<IS_BF16>(cur, b[i / DB], acc[i % DB]);
+      if (i < 8) {
+        kcopy(2 * i, next, na, nb);
+        kcopy(2 * i + 1, next, na, nb);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DB; ++i) pin_agpr(acc[i]);
+  };
+  if (steps > 0) {
+    copy_ds(0, S0);
+    copy_ds(1, S1);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) kcopy(i, key_of(0), K00, K01);
+  }
+  for (int s = 0; s + 1 < steps; s += 2) {
+    step(s, K00, K01, S0, K10, K11);
+    __builtin_amdgcn_sched_barrier(0);
+    step(s + 1, K10, K11, S1, K00, K01);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (steps & 1) step(steps - 1, K00, K01, S0, K10, K11);
+  drain_tile_copies();
+
+  // The groups' sums through their own tile buffers (two 4 KB blocks db in each; query row r at byte
+  // 128 r, 16-byte chunk c (4 columns) at c ^ ((r >> 1) & 7)), then each wave adds and stores
+  // a share of the rows, 8 rows x 64 columns per instruction, non-temporally. Accumulator column
+  // l32 is query sigma(l32) of the tile (gfa_ds.h).
+  const int ln = opaque(lane);
+  auto blk = [&](int db, int w) __attribute__((always_inline)) {
+    return (db < 2 ? (char GFA_LDS*)k_lds00 : db < 4 ? (char GFA_LDS*)k_lds01 : db < 6 ? (char GFA_LDS*)k_lds10
+                                                                               : (char GFA_LDS*)k_lds11) +
+           w * HALF + (db & 1) * 4096;
+  };
+  {
+    const int c8 = (ln & 31) >> 3, e8 = ln & 7;
+    const int r = 16 * (c8 >> 1) + 8 * (e8 >> 2) + 4 * (c8 & 1) + (e8 & 3);
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 o4 = {acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+        *reinterpret_cast<f32x4 GFA_LDS*>(blk(db, wave) + r * 128 + (((2 * g + (ln >> 5)) ^ ((r >> 1) & 7)) << 4)) = o4;
+      }
+    }
+  }
+  barrier_lds();
+  uint16_t* const ob = p.dq + (int64_t)b * p.dqv.sb + (int64_t)head * p.dqv.sh + DW * dh;
+#pragma unroll
+  for (int i = 0; i < 32 / NG / 8; ++i) {
+    const int r = grp * (32 / NG) + 8 * i + (ln >> 3);
+    const int sw = (r >> 1) & 7;
+    const int c0 = 2 * (ln & 3);
+#pragma unroll
+    for (int j = 0; j < DW / 64; ++j) {
+      f32x4 lo{}, hi{};
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const int w = g * SD + dh;
+        const char GFA_LDS* const src = ((ln >> 2) & 1) ? blk(2 * j + 1, w) : blk(2 * j, w);
+        lo += *reinterpret_cast<const f32x4 GFA_LDS*>(src + r * 128 + ((c0 ^ sw) << 4));
+        hi += *reinterpret_cast<const f32x4 GFA_LDS*>(src + r * 128 + (((c0 + 1) ^ sw) << 4));
+      }
+      i16x8 o8;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o8[e] = to16<IS_BF16>(lo[e] * p.scale);
+        o8[4 + e] = to16<IS_BF16>(hi[e] * p.scale);
+      }
+      const int q = qt * 32 + r;
+      if (q < p.N)
+        __builtin_nontemporal_store(o8, reinterpret_cast<i16x8*>(ob + (int64_t)q * p.dqv.sn + 64 * j + 8 * (ln & 7)));
+    }
+  }
+}
+
 #define GFA_DS_INST(DD, WW)                                                                   \
   template __global__ void bwd_dq_ds_kernel<DD, true, WW>(const BwdDqDsParams);               \
   template __global__ void bwd_dq_ds_kernel<DD, false, WW>(const BwdDqDsParams);              \
+  template __global__ void bwd_dq_rows_kernel<DD, true>(const BwdDqDsParams);                 \
+  template __global__ void bwd_dq_rows_kernel<DD, false>(const BwdDqDsParams);                \
   template __global__ void delta_kernel<DD, true>(const DeltaParams);                         \
   template __global__ void delta_kernel<DD, false>(const DeltaParams);
 GFA_DS_INST(512, 1)
@@ -443,6 +646,22 @@ hipError_t launch_delta(const DeltaParams& p, bool bf16, hipStream_t stream) {
   GFA_DELTA_CASE(512)
   GFA_DELTA_CASE(256)
 #undef GFA_DELTA_CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_bwd_dq_rows(const BwdDqDsParams& p, int head_dim, bool bf16, hipStream_t stream) {
+#define GFA_DQ_ROWS_CASE(DD)                                                                                      \
+  if (head_dim == DD) {                                                                                           \
+    if (bf16) {                                                                                                   \
+      hipLaunchKernelGGL((bwd_dq_rows_kernel<DD, true>), dim3(p.g.nblocks), dim3(256), 0, stream, p);             \
+    } else {                                                                                                      \
+      hipLaunchKernelGGL((bwd_dq_rows_kernel<DD, false>), dim3(p.g.nblocks), dim3(256), 0, stream, p);            \
+    }                                                                                                             \
+    return hipGetLastError();                                                                                     \
+  }
+  GFA_DQ_ROWS_CASE(512)
+  GFA_DQ_ROWS_CASE(256)
+#undef GFA_DQ_ROWS_CASE
   return hipErrorInvalidValue;
 }
 

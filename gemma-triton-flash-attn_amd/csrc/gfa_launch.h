@@ -18,6 +18,7 @@ hipError_t launch_seg_positions(const void* pos, bool is64, int64_t row_stride, 
                                 hipStream_t stream);
 hipError_t launch_seg_mask(const uint8_t* mask, int64_t row_stride, int B, int N, int* lo, int* hi, int* bad,
                            hipStream_t stream);
+hipError_t launch_bwd_dq_rows(const BwdDqDsParams& p, int head_dim, bool bf16, hipStream_t stream);
 hipError_t launch_bwd_dq_ds(const BwdDqDsParams& p, int head_dim, bool bf16, hipStream_t stream);
 
 }  // namespace gfa
