@@ -140,14 +140,14 @@ gfa::QGrid make_qgrid(int B, int Hkv, int R, int N, int nu) {
 // The forward kernel for small grids (gfa_fwd_rows.hip: one workgroup per 32 query rows, its
 // waves splitting the keys) where fwd_kernel's 128-row workgroups leave CUs idle and its time is
 // the longest row's serial walk. Counted in 32-row blocks, one resident workgroup per CU:
-// - up to 256 (one round): 1.5-1.6x faster at D=512 (8:1 N=1024 causal 50.7 -> 31.5 us), up to
-//   1.8x at D=256 and below (8:4 D=256 N=1024 30.0 -> 16.7 us). At D=64 a sequence of up to one
-//   128-key tile has nothing to split (5.2 -> 5.8 us) and stays;
+// - up to 256 (one round): 1.6x faster at D=512 (8:1 N=1024 causal 50.4 -> 30.5 us), up to
+//   2.0x at D=256 and below (8:4 D=256 N=1024 30.0 -> 15.1 us). At D=64 a sequence of up to one
+//   128-key tile has nothing to split (4.9 -> 5.6 us) and stays;
 // - up to 512 under full causal masking, whose second round is the short rows: D=512 8:1 N=2048
-//   90.7 -> 71.3, D=256 8:4 N=2048 54.1 -> 34.1, D=128 8:2 N=2048 35.4 -> 22.0 us; below D=256
-//   only from 1024 tokens (D=128 32:8 N=333 10.6 -> 11.8 us).
+//   90.3 -> 67.2, D=256 8:4 N=2048 53.5 -> 31.9, D=128 8:2 N=2048 35.3 -> 20.3 us; below D=256
+//   only from 1024 tokens (D=128 32:8 N=333 10.7 -> 11.1 us).
 // Past that the K / V copies per 32 rows cost more than the idle CUs (D=512 8:1 N=3000, 752
-// blocks: 128 -> 142 us; windows: D=256 8:1 W=512 N=1500, 376 blocks: 20.2 -> 23.5 us).
+// blocks: 126 -> 135 us; windows: D=256 8:1 W=512 N=1500, 376 blocks: 20.9 -> 22.1 us).
 // The dQ kernel of the materialised backward has the same two forms and the same line
 // (bwd_dq_rows_kernel against bwd_dq_ds_kernel): D=512 8:1 N=1024 31.6 -> 15.2 us, N=2000 57.2 -> 40.8,
 // 16:2 N=1300 (656 blocks) 42.8 -> 39.3, N=2048 (1024) 62.2 -> 75.0; D=256 8:4 N=2048 32.8 -> 24.2, N=3000

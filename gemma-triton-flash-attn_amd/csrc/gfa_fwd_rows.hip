@@ -12,10 +12,12 @@
 //  * A wave's tiles are private, so the loop has no workgroup barrier at D <= 256; at D = 512 the
 //    two waves of a pair add their halves of S once per tile (one barrier).
 //  * A tile is 8192 elements of K and of V per wave (32 keys at a width of 256, 64 at 128, 128 at
-//    64), in four cells each of 32 rows x 64 columns (4 KB, one LDS object per cell). A cell is
-//    consumed by four products; its refill (the next tile's cell, four 1 KB direct global->LDS
-//    copies) is issued one copy per product right behind it, so the copies run almost a whole
-//    tile ahead of their use out of a single-buffered tile.
+//    64), in two cells each of 32 rows x 128 columns (64 x 64 at D = 64; 8 KB, one LDS object per
+//    cell). A cell is consumed by eight products; its refill (the next tile's cell, eight 1 KB
+//    direct global->LDS copies) is issued one copy per product right behind it, so the copies
+//    run most of a tile ahead of their use out of a single-buffered tile. The copies' row
+//    pieces are 256 bytes: with 128-byte ones (cells of 64 columns) the kernel took 3-6% longer at
+//    D >= 256 (8:1 D=512 N=2048 causal 70.4 -> 66.4 us, 8:4 D=256 N=700 13.9 -> 12.8 us).
 // Bound: every wave reads its own K / V from L2, 32 rows of queries per tile byte (128 in
 // fwd_kernel), so with all CUs busy the copies (64 B per CU and clock) take twice the products'
 // time. The host takes this kernel where the 128-row grid leaves CUs idle (gfa_api.hip).
@@ -33,25 +35,30 @@ __device__ __forceinline__ void wait_copies() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Copies cells (32 rows x 64 columns of a row-major 16-bit slice) into LDS: row r at byte 128 r,
-// 16-byte chunk c at chunk position c ^ swz<64>(r). Four instructions of 8 whole 128-byte rows.
+// Copies cells (4096 elements: 4096 / CW rows x CW columns of a row-major 16-bit slice) into LDS: row r at
+// byte 2 CW r, 16-byte chunk c at chunk position c ^ swz<CW>(r). Eight instructions of whole row
+// pieces.
+template <int CW>
 struct CellLoader {
+  static constexpr int LPR = CW / 8;    // lanes per row piece
+  static constexpr int RPI = 64 / LPR;  // rows per instruction
+  static constexpr int NV = 16 / RPI;   // the swizzle repeats every 16 rows
   __amdgpu_buffer_rsrc_t rsrc;
-  unsigned voff[2];  // the swizzle repeats every 16 rows
+  unsigned voff[NV];
   unsigned stride_b;
   __device__ __forceinline__ void init(const uint16_t* base, int64_t row_stride, int n_rows, int row_elems, int lane) {
     stride_b = (unsigned)(row_stride * 2);
     rsrc = slice_rsrc(base, row_stride, n_rows, row_elems);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 8 * i + (lane >> 3);
-      voff[i] = (lane >> 3) * stride_b + (unsigned)(((lane & 7) ^ swz<64>(row)) << 4);
+    for (int i = 0; i < NV; ++i) {
+      const int row = RPI * i + lane / LPR;
+      voff[i] = (lane / LPR) * stride_b + (unsigned)(((lane % LPR) ^ swz<CW>(row)) << 4);
     }
   }
-  // Instruction i (< 4) of the cell at rows row0 .., columns from byte col_b of the row.
+  // Instruction i (< 8) of the cell at rows row0 .., columns from byte col_b of the row.
   __device__ __forceinline__ void load_part(int i, int row0, int col_b, char GFA_LDS* cell) const {
-    const unsigned soff = (unsigned)(row0 + 8 * i) * stride_b + (unsigned)col_b;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (void GFA_LDS*)(cell + i * 1024), 16, voff[i & 1], soff, 0, 0);
+    const unsigned soff = (unsigned)(row0 + RPI * i) * stride_b + (unsigned)col_b;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (void GFA_LDS*)(cell + i * 1024), 16, voff[i % NV], soff, 0, 0);
   }
 };
 
@@ -66,19 +73,21 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
   constexpr int KT = DW / 16;
   constexpr int DB = DW / 32;
   constexpr int SB = BKV / 32;
-  constexpr int CG = DW / 64;           // cells per 32 rows
-  constexpr int CELL = 4096;
+  constexpr int CW = DW < 128 ? DW : 128;  // cell: CR rows x CW columns
+  constexpr int CR = 4096 / CW;
+  constexpr int CG = DW / CW;           // cells side by side
+  constexpr int CELL = 8192;
   constexpr int PF = 4;                 // LDS read-ahead, in products
   constexpr float kMargin = IS_BF16 ? 64.0f : 15.0f;      // as fwd_kernel
   constexpr float kMaxRowSum = 18446744073709551616.0f;
   constexpr bool LAZY = IS_BF16;
-  static_assert(SB * KT == 16 && SB * 2 * DB == 16 && SB * CG == 4, "16 products and four cells per phase");
-  static_assert(PF == 4, "the copy counts below assume a read-ahead of one cell");
+  static_assert(SB * KT == 16 && SB * 2 * DB == 16 && BKV / CR * CG == 2, "16 products and two cells per phase");
+  static_assert(PF == 4, "the copy counts below assume a read-ahead of half a cell");
 
   // One LDS object per cell (the compiler tells a read of one cell from the copies in flight into
-  // the others), each with a 4 KB block per wave.
-  __shared__ __attribute__((aligned(1024))) char k0_lds[4 * CELL], k1_lds[4 * CELL], k2_lds[4 * CELL], k3_lds[4 * CELL];
-  __shared__ __attribute__((aligned(1024))) char v0_lds[4 * CELL], v1_lds[4 * CELL], v2_lds[4 * CELL], v3_lds[4 * CELL];
+  // the others), each with an 8 KB block per wave.
+  __shared__ __attribute__((aligned(1024))) char k0_lds[4 * CELL], k1_lds[4 * CELL];
+  __shared__ __attribute__((aligned(1024))) char v0_lds[4 * CELL], v1_lds[4 * CELL];
   // SD = 2: the pairs' S halves, double buffered (4 KB per wave). After the loop: row statistics.
   constexpr int PX = SD == 2 ? 2 * 4 * 4096 : 1024;
   __shared__ __attribute__((aligned(1024))) char x_lds[PX];
@@ -91,12 +100,10 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
   const int h = lane >> 5;
   const int l32 = lane & 31;
   auto kcell = [&](int c, int w) __attribute__((always_inline)) {
-    return (c == 0 ? (char GFA_LDS*)k0_lds : c == 1 ? (char GFA_LDS*)k1_lds : c == 2 ? (char GFA_LDS*)k2_lds
-                                                                             : (char GFA_LDS*)k3_lds) + w * CELL;
+    return (c == 0 ? (char GFA_LDS*)k0_lds : (char GFA_LDS*)k1_lds) + w * CELL;
   };
   auto vcell = [&](int c, int w) __attribute__((always_inline)) {
-    return (c == 0 ? (char GFA_LDS*)v0_lds : c == 1 ? (char GFA_LDS*)v1_lds : c == 2 ? (char GFA_LDS*)v2_lds
-                                                                             : (char GFA_LDS*)v3_lds) + w * CELL;
+    return (c == 0 ? (char GFA_LDS*)v0_lds : (char GFA_LDS*)v1_lds) + w * CELL;
   };
 
   // ---- workgroup -> (b, head, 32-row query block); the R heads of a KV head side by side on one
@@ -141,15 +148,15 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
   // a workgroup barrier); a group's tile past t_hi is fully masked and copies nothing.
   const int steps = SD == 2 ? (t_hi - t_lo + NG - 1) / NG : max(0, (t_hi - t_lo - grp + NG - 1) / NG);
 
-  CellLoader kload, vload;
+  CellLoader<CW> kload, vload;
   kload.init(p.k + (int64_t)b * p.kv.sb + (int64_t)kvh * p.kv.sh, p.kv.sn, p.N, D, lane);
   vload.init(p.v + (int64_t)b * p.vv.sb + (int64_t)kvh * p.vv.sh, p.vv.sn, p.N, D, lane);
   // Copy instruction i of cell c of the tile at row0.
   auto kcopy = [&](int c, int i, int row0) __attribute__((always_inline)) {
-    kload.load_part(i, row0 + 32 * (c / CG), 128 * (c % CG) + 2 * DW * dh, kcell(c, wave));
+    kload.load_part(i, row0 + CR * (c / CG), 2 * CW * (c % CG) + 2 * DW * dh, kcell(c, wave));
   };
   auto vcopy = [&](int c, int i, int row0) __attribute__((always_inline)) {
-    vload.load_part(i, row0 + 32 * (c / CG), 128 * (c % CG) + 2 * DW * dh, vcell(c, wave));
+    vload.load_part(i, row0 + CR * (c / CG), 2 * CW * (c % CG) + 2 * DW * dh, vcell(c, wave));
   };
   // First row of step s's tile; rows past the sequence end (no such tile) copy zeros, no memory read.
   auto row_of = [&](int s) __attribute__((always_inline)) {
@@ -165,24 +172,26 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     for (int kk = 0; kk < KT; ++kk) qf[kk] = *reinterpret_cast<const i16x8*>(qp + 16 * kk);
   }
 
-  // Per-lane LDS offsets inside a cell: K row l32 at chunk 2 (kk & 3) + h; V read transposed (rows
-  // 4h + t/4 and 8 further, column block db & 1). As kstep_off / mma_tr_accumulate_b at D = 64.
-  const int koff0 = l32 * 128 + ((h ^ swz<64>(l32)) << 4);
+  // Per-lane LDS offsets inside a cell: K row l32 at chunk 2 kk + h; V read transposed (rows 4h + t/4
+  // and 8 further, column block 0). As kstep_off / mma_tr_accumulate_b at D = CW.
+  const int koff0 = l32 * (2 * CW) + ((h ^ swz<CW>(l32)) << 4);
   int voff0;
   {
     const int t16 = lane & 15;
     const int rA = 4 * h + (t16 >> 2);
     const int c = 2 * ((lane >> 4) & 1) + ((t16 >> 1) & 1);
-    voff0 = rA * 128 + ((c ^ swz<64>(rA)) << 4) + (t16 & 1) * 8;
+    voff0 = rA * (2 * CW) + ((c ^ swz<CW>(rA)) << 4) + (t16 & 1) * 8;
   }
-  // A operand of S product i (key block i / KT, k-step i % KT; cell i / 4) and of PV product i: cell
-  // i / 4 = (key block, column group), then k-step (i >> 1) & 1, column block i & 1.
+  // A operand of S product i (key block i / KT, k-step i % KT; cell i / 8) and of PV product i: cell
+  // i / 8, then the k-steps of its rows, then its column blocks.
   auto kfrag = [&](int i) __attribute__((always_inline)) {
-    return lds_read16(kcell(i >> 2, wave), koff0 ^ ((i & 3) << 5));
+    const int kk = i % (CW / 16), rb = (i & 7) / (CW / 16);  // k-step, 32-row block inside the cell
+    return lds_read16(kcell(i >> 3, wave), (koff0 ^ (kk << 5)) + rb * 32 * (2 * CW));
   };
+  constexpr int CB = CW / 32;  // column blocks per cell
   auto vfrag = [&](int i) __attribute__((always_inline)) {
-    const int a = (voff0 ^ ((i & 1) << 6));
-    return tr_frag(vcell(i >> 2, wave), a, (a ^ 32) + 1024, ((i >> 1) & 1) * 2048);
+    const int a = voff0 ^ ((i % CB) << 6);
+    return tr_frag(vcell(i >> 3, wave), a, (a ^ 32) + 16 * CW, ((i & 7) / CB) * 16 * (2 * CW));
   };
 
   f32x16 acc[DB];
@@ -200,7 +209,7 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     for (int i = 0; i < 16; ++i) {
       const i16x8 cur = a[i % PF];
       if (i + PF < 16) {
-        if (i % 4 == 0) wait_copies<20>();
+        if (i + PF == 8) wait_copies<12>();
         a[i % PF] = kfrag(i + PF);
       }
       // in VGPRs (O^T is pinned to AGPRs; see mma32_vgpr)
@@ -259,10 +268,11 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     return halves_max(m) * xs;
   };
 
-  // One pass over the group's tiles. Cells are consumed in the order K0..K3, V0..V3; behind
-  // cell c's products go the four copies that refill cell c - 1 with the next tile (V3 behind
-  // K0, K3 behind V0). Before a phase's first read the copies issued after its first cell are
-  // six cells' (24 instructions), before the reads of its next cells five cells' (20).
+  // One pass over the group's tiles. Cells are consumed in the order K0, K1, V0, V1; behind a cell's
+  // products go the eight copies that refill the cell before it with the next tile (V1 behind K0,
+  // K1 behind V0). Before a phase's first read the copies issued after its first cell are two
+  // cells' (16 instructions), before the first read of its second cell (PF products ahead) one and
+  // a half's (12).
   auto run_pass = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < DB; ++i) acc[i] = f32x16{};
@@ -270,30 +280,30 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     int row = row_of(0);
     if (steps > 0) {
 #pragma unroll
-      for (int c = 0; c < 7; ++c) {
+      for (int c = 0; c < 3; ++c) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (c < 4) {
+        for (int i = 0; i < 8; ++i) {
+          if (c < 2) {
             kcopy(c, i, row);
           } else {
-            vcopy(c - 4, i, row);
+            vcopy(0, i, row);
           }
         }
       }
-    }
-    // The Q loads complete here, ahead of the copies in flight (left to the loop's first use, the
-    // compiler drains every copy before the loop).
+      // The Q loads complete here, ahead of the copies in flight (left to the loop's first use, the
+      // compiler drains every copy before the loop).
 #pragma unroll
-    for (int kk = 0; kk < KT; ++kk) pin_vgpr(qf[kk]);
+      for (int kk = 0; kk < KT; ++kk) pin_vgpr(qf[kk]);
+    }
     for (int s = 0; s < steps; ++s) {
       const int next = row_of(s + 1);
       f32x16 sc[SB];
-      wait_copies<24>();
+      wait_copies<16>();
       scores(s, sc, [&](int i) __attribute__((always_inline)) {
-        if (i < 4) {
-          vcopy(3, i, row);
+        if (i < 8) {
+          vcopy(1, i, row);
         } else {
-          kcopy((i >> 2) - 1, i & 3, next);
+          kcopy(0, i - 8, next);
         }
       });
       if (!LAZY || __builtin_amdgcn_ballot_w64(m_ref == kNegBig) != 0) {
@@ -319,24 +329,24 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
           pb[sb * 2 + (r >> 3)][r & 7] = to16<IS_BF16>(pk);
         }
       }
-      wait_copies<24>();
+      wait_copies<16>();
       i16x8 a[PF];
 #pragma unroll
       for (int i = 0; i < PF; ++i) a[i] = vfrag(i);
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int rb = (i >> 2) / CG, cg = (i >> 2) % CG;
-        const int ks = 2 * rb + ((i >> 1) & 1), db = 2 * cg + (i & 1);
+        const int rb = (i >> 3) / CG, cg = (i >> 3) % CG;
+        const int ks = CR / 16 * rb + (i & 7) / CB, db = CB * cg + i % CB;
         const i16x8 cur = a[i % PF];
         if (i + PF < 16) {
-          if (i % 4 == 0) wait_copies<20>();
+          if (i + PF == 8) wait_copies<12>();
           a[i % PF] = vfrag(i + PF);
         }
         acc[db] = mma32<IS_BF16>(cur, pb[ks], acc[db]);
-        if (i < 4) {
-          kcopy(3, i, next);
+        if (i < 8) {
+          kcopy(1, i, next);
         } else {
-          vcopy((i >> 2) - 1, i & 3, next);
+          vcopy(0, i - 8, next);
         }
       }
 #pragma unroll
@@ -378,9 +388,9 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
       for (int s = 0; s < steps; ++s) {
         const int row = row_of(s);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 2; ++c) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) kcopy(c, i, row);
+          for (int i = 0; i < 8; ++i) kcopy(c, i, row);
         }
         wait_copies<0>();
         f32x16 sc[SB];
@@ -408,11 +418,13 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
   if (p.store_lse && wave == 0 && h == 0 && q < p.N)
     p.lse[((int64_t)b * p.Hq + head) * p.lse_ld + q] = (m_tot + __log2f(l_tot)) * kLn2;
 
-  // This wave's normalised O (fp32) into its own cells: accumulator block db in cell db (K0..K3,
-  // V0..V3), row r at byte 128 r, 16-byte chunk c (4 columns) at c ^ ((r >> 1) & 7).
+  // This wave's normalised O (fp32) into its own cells: two 4 KB accumulator blocks db per cell (K0,
+  // K1, V0, V1), row r at byte 128 r, 16-byte chunk c (4 columns) at c ^ ((r >> 1) & 7).
   const int ln = opaque(lane);
   const int r32 = ln & 31;
-  auto cell = [&](int c, int w) __attribute__((always_inline)) { return c < 4 ? kcell(c, w) : vcell(c - 4, w); };
+  auto cell = [&](int db, int w) __attribute__((always_inline)) {
+    return (db < 4 ? kcell(db >> 1, w) : vcell((db >> 1) - 2, w)) + (db & 1) * 4096;
+  };
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
 #pragma unroll
@@ -431,7 +443,7 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     const int sw = (r >> 1) & 7;
     const int c0 = 2 * (ln & 3);
 #pragma unroll
-    for (int j = 0; j < CG; ++j) {
+    for (int j = 0; j < DW / 64; ++j) {
       f32x4 lo{}, hi{};
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
@@ -452,6 +464,23 @@ __global__ __launch_bounds__(256, 1) void fwd_rows_kernel(const FwdParams p) {
     }
   }
 }
+
+// Explicit instantiations of every built variant (device code and host launch stubs).
+#define GFA_ROWS_INST(DD, CC, XX)                                                     \
+  template __global__ void fwd_rows_kernel<DD, true, false, CC, XX>(const FwdParams);  \
+  template __global__ void fwd_rows_kernel<DD, false, false, CC, XX>(const FwdParams); \
+  template __global__ void fwd_rows_kernel<DD, true, true, CC, XX>(const FwdParams);   \
+  template __global__ void fwd_rows_kernel<DD, false, true, CC, XX>(const FwdParams);
+#define GFA_ROWS_INST_D(DD)       \
+  GFA_ROWS_INST(DD, false, false) \
+  GFA_ROWS_INST(DD, true, false)  \
+  GFA_ROWS_INST(DD, false, true)
+GFA_ROWS_INST_D(512)
+GFA_ROWS_INST_D(256)
+GFA_ROWS_INST_D(128)
+GFA_ROWS_INST_D(64)
+#undef GFA_ROWS_INST_D
+#undef GFA_ROWS_INST
 
 template <int D, bool IS_BF16, bool CAP, bool DROP>
 static hipError_t launch_rows_t(const FwdParams& p, hipStream_t stream) {

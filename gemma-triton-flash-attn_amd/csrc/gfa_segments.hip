@@ -144,6 +144,9 @@ __global__ __launch_bounds__(kTpb) void seg_mask_kernel(const uint8_t* mask, int
   if (blockIdx.x == 0 && tid == 0) bad[blockIdx.y] = count > 0 && count != end - start;
 }
 
+template __global__ void seg_positions_kernel<int64_t>(const int64_t*, int64_t, int, int*, int*);
+template __global__ void seg_positions_kernel<int32_t>(const int32_t*, int64_t, int, int*, int*);
+
 hipError_t launch_seg_positions(const void* pos, bool is64, int64_t row_stride, int B, int N, int* lo, int* hi,
                                 hipStream_t stream) {
   const dim3 grid((N + kTpb - 1) / kTpb, B);
