@@ -137,26 +137,40 @@ gfa::QGrid make_qgrid(int B, int Hkv, int R, int N, int nu) {
   return g;
 }
 
-// The forward kernel for small grids (gfa_fwd_rows.hip: one workgroup per 32 query rows, its
-// waves splitting the keys) where fwd_kernel's 128-row workgroups leave CUs idle and its time is
-// the longest row's serial walk. Counted in 32-row blocks, one resident workgroup per CU:
-// - up to 256 (one round): 1.6x faster at D=512 (8:1 N=1024 causal 50.4 -> 30.5 us), up to
+// The kernels for small grids (forward: gfa_fwd_rows.hip, one workgroup per 32 query rows, its
+// waves splitting the keys; dQ of the materialised backward: bwd_dq_rows_kernel) where the
+// 128-row workgroups of fwd_kernel / bwd_dq_ds_kernel leave CUs idle and the time is the longest
+// row's serial walk. Counted in 32-row blocks, one resident workgroup per CU:
+// - up to 256 (one round): forward 1.6x faster at D=512 (8:1 N=1024 causal 50.4 -> 30.5 us), up to
 //   2.0x at D=256 and below (8:4 D=256 N=1024 30.0 -> 15.1 us). At D=64 a sequence of up to one
-//   128-key tile has nothing to split (4.9 -> 5.6 us) and stays;
-// - up to 512 under full causal masking, whose second round is the short rows: D=512 8:1 N=2048
-//   90.3 -> 67.2, D=256 8:4 N=2048 53.5 -> 31.9, D=128 8:2 N=2048 35.3 -> 20.3 us; below D=256
-//   only from 1024 tokens (D=128 32:8 N=333 10.7 -> 11.1 us).
-// Past that the K / V copies per 32 rows cost more than the idle CUs (D=512 8:1 N=3000, 752
-// blocks: 126 -> 135 us; windows: D=256 8:1 W=512 N=1500, 376 blocks: 20.9 -> 22.1 us).
-// The dQ kernel of the materialised backward has the same two forms and the same line
-// (bwd_dq_rows_kernel against bwd_dq_ds_kernel): D=512 8:1 N=1024 31.6 -> 15.2 us, N=2000 57.2 -> 40.8,
-// 16:2 N=1300 (656 blocks) 42.8 -> 39.3, N=2048 (1024) 62.2 -> 75.0; D=256 8:4 N=2048 32.8 -> 24.2, N=3000
-// (752) 46.0 -> 49.0; window 512 8:1 N=800 (200) 13.6 -> 9.2, N=2000 (504) 14.3 -> 17.1.
+//   128-key tile has nothing to split (4.9 -> 5.6 us) and stays. dQ: D=512 8:1 N=1024 31.6 -> 15.2 us;
+// - up to 512 under full causal masking, whose second round is the short rows: forward D=512 8:1
+//   N=2048 90.3 -> 67.2, D=256 8:4 N=2048 53.5 -> 31.9, D=128 8:2 N=2048 35.3 -> 20.3 us, dQ D=512
+//   8:1 N=2000 57.2 -> 40.8, D=256 8:4 N=2048 32.8 -> 24.2; below D=512 only where a row is long enough
+//   to split (forward 16:4 N=608 D=256 20.5 -> 16.6, D=64 10.3 -> 9.8; 4 rows of 8:4 N=320 D=256
+//   13.3 -> 15.2, N=416 D=256 dQ 11.2 -> 12.4, N=512 D=64 9.2 -> 10.5).
+// Past that the K / V copies (dS and K for dQ) per 32 rows cost more than the idle CUs: D=512 8:1
+// N=3000, 752 blocks, forward 126 -> 135 us, dQ D=256 8:4 N=3000 46.0 -> 49.0; windows: D=256 8:1 W=512
+// N=1500, 376 blocks, forward 20.9 -> 22.1 us.
 bool use_rows_kernel(int D, int B, int Hq, int N, bool causal, bool windowed) {
   const long long blocks = (long long)B * Hq * ((N + 31) / 32);
   if (D == 64 && N <= 128) return false;
   if (blocks <= 256) return true;
-  return blocks <= 512 && causal && !windowed && (D >= 256 || N >= 1024);
+  return blocks <= 512 && causal && !windowed && (D == 512 || N >= 640);
+}
+
+// The forward below D=512 crosses later the longer the walk, where no window or segment table cuts it short:
+// - causal, up to 768 blocks from 2048 tokens (D=256 8:4 N=3072 77.5 -> 64.3 us, D=64 4:1 N=6144
+//   66.7 -> 40.3; 16:4 N=1536 D=64 19.9 -> 19.9), up to 1024 from 4096 (D=256 8:4 N=4096 103.3 -> 102.3,
+//   D=128 65.5 -> 58.7, 4:1 N=8192 126.3 -> 97.2; 16:4 N=2048 D=256 55.0 -> 63.9);
+// - without a mask, up to 512 blocks from 1536 tokens (8:4 N=2048 D=256 54.3 -> 51.6, D=64 24.8 -> 19.8;
+//   16:4 N=1024 D=256 30.3 -> 32.0; 576 blocks, 8:4 D=256 60.4 -> 78.0).
+bool use_rows_forward(int D, int B, int Hq, int N, bool causal, bool windowed, bool segments) {
+  if (use_rows_kernel(D, B, Hq, N, causal, windowed)) return true;
+  if (D == 512 || windowed || segments) return false;
+  const long long blocks = (long long)B * Hq * ((N + 31) / 32);
+  if (causal) return N >= 2048 && blocks <= (N >= 4096 ? 1024 : 768);
+  return N >= 1536 && blocks <= 512;
 }
 
 gfa::QGrid rows_grid(int B, int Hkv, int R, int N) {
@@ -517,7 +531,7 @@ int gfa_fwd(const gfa_fwd_args* a) {
   if (p.store_lse && (a->lse_ld < GFA_LSE_LD(a->seq_len) || !aligned16(a->lse) || (a->lse_ld & 3)))
     return fail(GFA_ERR_INVALID_ARGUMENT, "lse_ld=%d must be >= %d (multiple of 4, 16-byte aligned lse)", a->lse_ld,
                 GFA_LSE_LD(a->seq_len));
-  if (a->block_kv == 0 && use_rows_kernel(a->head_dim, p.B, p.Hq, p.N, p.causal, windowed)) {
+  if (a->block_kv == 0 && use_rows_forward(a->head_dim, p.B, p.Hq, p.N, p.causal, windowed, a->seg_lo != nullptr)) {
     p.g = rows_grid(p.B, p.Hkv, p.R, p.N);
     const hipError_t err = gfa::launch_fwd_rows(p, a->head_dim, a->dtype == GFA_DTYPE_BF16, cap, drop,
                                                 static_cast<hipStream_t>(a->stream));

@@ -2,7 +2,7 @@
 general one (fwd_kernel, which an explicit ``block_kv`` always runs) and against the oracle.
 
 Sizes sit at the edges of its tiles (32, 64 and 128 keys per wave at head dims 256 and 512, 128, 64;
-32-row blocks; two or four key groups) and of the rule that selects it (256 and 512 row blocks).
+32-row blocks; two or four key groups) and of the rule that selects it (256 to 1024 row blocks).
 
 Both forwards round P to the 16-bit type before P V (unit roundoff u = 2^-8 in bf16, 2^-11 in fp16,
 relative to P, against their own reference max) and O at the end, so with A = softmax |V| they
@@ -101,7 +101,17 @@ def test_features(D, N, causal, window, feature, dtype, device):
     (1, 8, 1, 1000, 256, True, 512),
     (2, 4, 4, 1024, 64, True, 0),
     (1, 16, 4, 1024, 128, True, 0),
-    (1, 16, 4, 1023, 128, True, 0),    # below 1024 tokens at 512 blocks: the general forward
+    (1, 16, 4, 1023, 128, True, 0),
+    (3, 8, 2, 640, 128, True, 0),      # 480 blocks
+    (3, 8, 2, 639, 128, True, 0),      # below 640 tokens: the general forward
+    (1, 8, 4, 3072, 256, True, 0),     # 768: the last below 4096 tokens
+    (1, 8, 4, 3073, 256, True, 0),
+    (1, 8, 4, 4095, 64, True, 0),      # 1024 blocks, one token short
+    (1, 8, 4, 4096, 128, True, 0),     # 1024, from 4096 tokens
+    (1, 4, 1, 8100, 64, True, 0),
+    (1, 8, 4, 2048, 64, False, 0),     # 512, no mask
+    (1, 5, 5, 1537, 256, False, 0),
+    (2, 4, 4, 2049, 128, False, 0),
 ])
 def test_rule_edges(B, Hq, Hkv, N, D, causal, window, device):
     _compare(B, Hq, Hkv, N, D, causal, window, torch.bfloat16, device, oracle=False)
