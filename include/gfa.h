@@ -210,7 +210,8 @@ int64_t gfa_bwd_ds_limit(int64_t bytes);
 /* Fill *out with the configuration used for this problem without a sliding window (with a
  * window shorter than the sequence, the forward at head_dim 128 runs 32-key tiles, and the
  * dK/dV kernel at head_dim 256 runs role-split wave pairs, 64 keys per workgroup, two
- * workgroups per CU; gfa_bwd_workspace_size reports the split count for either). Returns a
+ * workgroups per CU; gfa_bwd_workspace_size reports the split count for either; grids too small
+ * to fill the GPU run 32-row workgroups in the forward and in dQ from the dS store). Returns a
  * gfa_status. */
 int gfa_config(int32_t batch, int32_t heads_q, int32_t heads_kv, int32_t seq_len, int32_t head_dim,
                gfa_config_info* out);
