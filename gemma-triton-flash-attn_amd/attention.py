@@ -327,8 +327,9 @@ def _native_call(q, k, v) -> bool:
 _ORDINARY = (torch.Tensor, torch.nn.Parameter)
 
 
-def _attend(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p, grad: bool):
-    """The C++ host path after the checks of FlashAttnGQAFunction.forward; ``grad``: with autograd."""
+def _attend(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p, grad: bool, as_op: bool = False):
+    """The C++ host path after the checks of FlashAttnGQAFunction.forward; ``grad``: with autograd
+    (``as_op``: the registered op's, whose gradients refuse to be differentiated again)."""
     _check_inputs(q, k, v)
     segments = _check_segments(segments, q)
     window = _norm_window(causal, slide_size, q.shape[2])
@@ -339,7 +340,7 @@ def _attend(q, k, v, causal, slide_size, scale, segments, softcap, dropout_p, gr
     seed = _dropout_seed() if dp > 0.0 else 0
     lo, hi = segments if segments is not None else (None, None)
     if grad:
-        return _lib.native().train(q, k, v, bool(causal), window, sc, cap, dp, seed, lo, hi)
+        return _lib.native().train(q, k, v, bool(causal), window, sc, cap, dp, seed, lo, hi, as_op)
     return _lib.native().infer(q, k, v, bool(causal), window, sc, cap, dp, seed, 0, lo, hi)
 
 

@@ -13,6 +13,7 @@
 // this call's tensors is decided here, by attention.py's rules: copies of inputs whose layout the
 // ABI cannot address, outputs in the input's layout where it can. Nothing is kept between calls.
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
@@ -84,7 +85,8 @@ struct Options {
   int64_t window;
   double scale, softcap, dropout_p;
   int64_t seed, block_kv;
-  Tensor lo, hi;  // segment tables, or undefined
+  Tensor lo, hi;       // segment tables, or undefined
+  bool as_op = false;  // autograd as the registered op's (Attention)
 };
 
 // O, and the LSE where asked for, of prepared inputs.
@@ -128,15 +130,58 @@ std::pair<Tensor, Tensor> forward_call(const Tensor& q, const Tensor& k, const T
   return {o, lse};
 }
 
+// Whether something stands between the engine and the tensors of a backward that a launch on their
+// pointers would pass by: compiled autograd's or a subclass's stand-ins for them, batched
+// gradients, a dispatch mode, a trace.
+bool watched(const Tensor& t) {
+  using c10::DispatchKey;
+  constexpr c10::DispatchKeySet keys({DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::FuncTorchBatched,
+                                      DispatchKey::FuncTorchGradWrapper, DispatchKey::Batched});
+  return t.key_set().has_any(keys);
+}
+bool watched(const torch::autograd::variable_list& tensors) {
+  using c10::DispatchKey;
+  for (const auto key : {DispatchKey::Python, DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::Tracer})
+    if (c10::impl::tls_is_dispatch_key_included(key)) return true;
+  for (const Tensor& t : tensors)
+    if (t.defined() && watched(t)) return true;
+  return false;
+}
+
+// dQ, dK, dV through the registered op gfa::attn_bwd (ops.py).
+std::tuple<Tensor, Tensor, Tensor> backward_op(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                               const Tensor& lse, const Tensor& dout, const Options& x,
+                                               const Tensor& seed) {
+  using Maybe = std::optional<Tensor>;
+  static const auto op =
+      c10::Dispatcher::singleton()
+          .findSchemaOrThrow("gfa::attn_bwd", "")
+          .typed<std::tuple<Tensor, Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                                                    const Tensor&, const Tensor&, bool, c10::SymInt, double,
+                                                    const Maybe&, const Maybe&, double, double, const Maybe&)>();
+  const auto maybe = [](const Tensor& t) { return t.defined() ? Maybe(t) : Maybe(); };
+  return op.call(q, k, v, o, lse, dout, x.causal, x.window, x.scale, maybe(x.lo), maybe(x.hi), x.softcap, x.dropout_p,
+                 maybe(seed));
+}
+
+// The autograd node of a call. With as_op (the transformers adapter, which is the registered op
+// gfa::attn_fwd everywhere else) a backward that itself records a graph (create_graph) calls the
+// op gfa::attn_bwd too: its gradients then refuse to be differentiated again, where the launch
+// below would give gradients without a graph and drop the second-order terms. Any watched
+// backward calls that op as well, so compiled autograd traces it into its one graph.
 struct Attention : public torch::autograd::Function<Attention> {
+  static constexpr bool is_traceable = true;
+
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v,
                         const Options& x) {
     auto [o, lse] = forward_call(prep(q), prep(k), prep(v), x, true);
-    if (x.lo.defined()) {
-      ctx->save_for_backward({q, k, v, o, lse, x.lo, x.hi});
-    } else {
-      ctx->save_for_backward({q, k, v, o, lse});
-    }
+    torch::autograd::variable_list saved{q, k, v, o, lse};
+    if (x.lo.defined()) saved.insert(saved.end(), {x.lo, x.hi});
+    // As the op does, a one-element CPU tensor: a compiled backward takes another seed each time.
+    if (x.as_op && x.dropout_p > 0.0) saved.push_back(at::full({1}, x.seed, at::kLong));
+    ctx->save_for_backward(std::move(saved));
+    ctx->saved_data["as_op"] = x.as_op;
+    ctx->saved_data["segments"] = x.lo.defined();
     ctx->saved_data["causal"] = x.causal;
     ctx->saved_data["window"] = x.window;
     ctx->saved_data["scale"] = x.scale;
@@ -149,8 +194,24 @@ struct Attention : public torch::autograd::Function<Attention> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  const torch::autograd::variable_list& grads) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor q = prep(saved[0]), k = prep(saved[1]), v = prep(saved[2]);
     const Tensor &o = saved[3], &lse = saved[4];
+    Options x{ctx->saved_data["causal"].toBool(),      ctx->saved_data["window"].toInt(),
+              ctx->saved_data["scale"].toDouble(),     ctx->saved_data["softcap"].toDouble(),
+              ctx->saved_data["dropout_p"].toDouble(), ctx->saved_data["seed"].toInt()};
+    x.as_op = ctx->saved_data["as_op"].toBool();
+    if (ctx->saved_data["segments"].toBool()) {
+      x.lo = saved[5];
+      x.hi = saved[6];
+    }
+    Tensor seed;
+    if (x.dropout_p > 0.0 && x.as_op) seed = saved.back();
+    if ((x.as_op && at::GradMode::is_enabled()) || watched(grads) || watched(saved)) {
+      if (x.dropout_p > 0.0 && !x.as_op) seed = at::full({1}, x.seed, at::kLong);
+      auto [dq, dk, dv] = backward_op(saved[0], saved[1], saved[2], o, lse, grads[0], x, seed);
+      return {dq, dk, dv, Tensor()};
+    }
+    if (seed.defined()) x.seed = seed.item<int64_t>();
+    const Tensor q = prep(saved[0]), k = prep(saved[1]), v = prep(saved[2]);
     const c10::DeviceGuard guard(q.device());
     Tensor dout = prep(grads[0]);
     if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
@@ -180,18 +241,18 @@ struct Attention : public torch::autograd::Function<Attention> {
     a.heads_kv = (int32_t)k.size(1);
     a.seq_len = (int32_t)q.size(2);
     a.head_dim = (int32_t)q.size(3);
-    a.causal = ctx->saved_data["causal"].toBool();
-    a.window = (int32_t)ctx->saved_data["window"].toInt();
-    a.scale = (float)ctx->saved_data["scale"].toDouble();
+    a.causal = x.causal;
+    a.window = (int32_t)x.window;
+    a.scale = (float)x.scale;
     a.dtype = dtype_of(q);
     a.lse_ld = (int32_t)lse.size(2);
-    a.softcap = (float)ctx->saved_data["softcap"].toDouble();
-    a.dropout_p = (float)ctx->saved_data["dropout_p"].toDouble();
-    a.dropout_seed = (uint64_t)ctx->saved_data["seed"].toInt();
+    a.softcap = (float)x.softcap;
+    a.dropout_p = (float)x.dropout_p;
+    a.dropout_seed = (uint64_t)x.seed;
     a.stream = stream_of(q);
-    if (saved.size() > 5) {
-      a.seg_lo = static_cast<const int32_t*>(saved[5].data_ptr());
-      a.seg_hi = static_cast<const int32_t*>(saved[6].data_ptr());
+    if (x.lo.defined()) {
+      a.seg_lo = static_cast<const int32_t*>(x.lo.data_ptr());
+      a.seg_hi = static_cast<const int32_t*>(x.hi.data_ptr());
     }
     Tensor ws;
     const size_t need = api.workspace_bytes(&a);
@@ -237,9 +298,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("train", torch::wrap_pybind_function(
                      [or_undefined](const Tensor& q, const Tensor& k, const Tensor& v, bool causal, int64_t window,
                                     double scale, double softcap, double dropout_p, int64_t seed,
-                                    const std::optional<Tensor>& lo, const std::optional<Tensor>& hi) {
+                                    const std::optional<Tensor>& lo, const std::optional<Tensor>& hi, bool as_op) {
                        const Options x{causal, window, scale, softcap, dropout_p, seed, 0,
-                                       or_undefined(lo), or_undefined(hi)};
+                                       or_undefined(lo), or_undefined(hi), as_op};
                        return Attention::apply(q, k, v, x);
                      }));
   // (lo, hi) tables, int32 (batch, seq_len), of unit-stride position ids (rows of stride 0 included).

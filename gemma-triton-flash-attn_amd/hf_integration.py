@@ -104,7 +104,7 @@ def triton_gqa_attention(module, query, key, value, attention_mask, dropout: flo
         drop = float(dropout or 0.0)
         if _native_call(query, key, value):
             grad = torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad)
-            out = _attend(query, key, value, is_causal, slide, scale, segments, softcap, drop, grad)
+            out = _attend(query, key, value, is_causal, slide, scale, segments, softcap, drop, grad, as_op=True)
         else:
             out = flash_attn_gqa_op(query, key, value, causal=is_causal, slide_size=slide, scale=scale,
                                     segments=segments, softcap=softcap, dropout_p=drop)
