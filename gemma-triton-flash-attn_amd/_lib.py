@@ -149,6 +149,15 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+def plain_setting() -> bool:
+    """Whether a call runs outside compilation, tracing, function transforms and modes (of dispatch or
+    of torch functions), all of which see tensor operations and registered ops but no launch on
+    their pointers."""
+    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None)
+
+
 _native = None
 
 

@@ -316,12 +316,9 @@ class FlashAttnGQAFunction(torch.autograd.Function):
 
 def _native_call(q, k, v) -> bool:
     """Whether a call takes the C++ host path (_lib.native(): the same launches, allocations and
-    autograd formula as below, without the interpreter): ordinary tensors, outside compilation,
-    tracing, function transforms and dispatch modes, which see the Python autograd function or the
-    registered op as before."""
-    return (type(q) in _ORDINARY and type(k) in _ORDINARY and type(v) in _ORDINARY
-            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._functorch.peek_interpreter_stack() is None)
+    autograd formula as below, without the interpreter): ordinary tensors in a plain setting. Any
+    other call goes through the Python autograd function or the registered op."""
+    return type(q) in _ORDINARY and type(k) in _ORDINARY and type(v) in _ORDINARY and _lib.plain_setting()
 
 
 _ORDINARY = (torch.Tensor, torch.nn.Parameter)

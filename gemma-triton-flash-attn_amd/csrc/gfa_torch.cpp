@@ -15,6 +15,7 @@
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -89,10 +90,12 @@ struct Options {
   bool as_op = false;  // autograd as the registered op's (Attention)
 };
 
-// O, and the LSE where asked for, of prepared inputs.
+// O, and the LSE where asked for, of prepared inputs. Profilers list it, and the backward below, under
+// the registered ops' names.
 std::pair<Tensor, Tensor> forward_call(const Tensor& q, const Tensor& k, const Tensor& v, const Options& x,
                                        bool store_lse) {
-  const c10::DeviceGuard guard(q.device());
+  RECORD_FUNCTION("gfa::attn_fwd", c10::ArrayRef<const c10::IValue>{});
+  const c10::DeviceGuard on_device(q.device());
   Tensor o = out_like(q);
   const int64_t ld = lse_ld(q.size(2));
   Tensor lse;
@@ -210,9 +213,10 @@ struct Attention : public torch::autograd::Function<Attention> {
       auto [dq, dk, dv] = backward_op(saved[0], saved[1], saved[2], o, lse, grads[0], x, seed);
       return {dq, dk, dv, Tensor()};
     }
+    RECORD_FUNCTION("gfa::attn_bwd", c10::ArrayRef<const c10::IValue>{});
     if (seed.defined()) x.seed = seed.item<int64_t>();
     const Tensor q = prep(saved[0]), k = prep(saved[1]), v = prep(saved[2]);
-    const c10::DeviceGuard guard(q.device());
+    const c10::DeviceGuard on_device(q.device());
     Tensor dout = prep(grads[0]);
     if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
     Tensor dq = out_like(q), dk = out_like(k), dv = out_like(v);

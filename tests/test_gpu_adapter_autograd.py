@@ -7,6 +7,7 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from conftest import make_inputs
@@ -119,3 +120,30 @@ def test_compiled_autograd(entry, feature, device):
         with torch._dynamo.compiled_autograd._enable(torch.compile(backend="aot_eager", fullgraph=True)):
             o.backward(do)
         assert all(torch.equal(x.grad, b) for x, b in zip(t, want))
+
+
+class _SeenFunctions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_function_modes_and_profiler(grad, device):
+    """A torch-function mode sees the op, and a profiler lists it by name, with and without gradients."""
+    t, do = _inputs(device)
+    with torch.set_grad_enabled(grad):
+        with _SeenFunctions() as seen:
+            out = _adapter(t, {})
+        assert any("gfa.attn_fwd" in n for n in seen.names)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            again = _adapter(t, {})
+            if grad:
+                again.backward(do)
+    assert torch.equal(out, again)
+    names = {e.key for e in prof.key_averages()}
+    assert "gfa::attn_fwd" in names and ("gfa::attn_bwd" in names) == grad
