@@ -54,11 +54,10 @@ def _host_checks() -> bool:
 
 def _native(t: torch.Tensor) -> bool:
     """Whether a table is built from ``t`` by the library's kernel (one launch): an ordinary tensor
-    on a GPU, outside tracing, function transforms and dispatch modes (which the tensor
-    operations below go through)."""
+    on a GPU in a plain setting. A trace, a transform or a mode goes through the tensor operations
+    below (a launch on pointers would freeze a traced batch's table into the trace)."""
     return (type(t) is torch.Tensor and t.is_cuda and t.dim() == 2 and t.numel() > 0 and t.shape[0] <= 65535
-            and _host_checks() and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and torch._C._len_torch_dispatch_stack() == 0)
+            and _lib.plain_setting() and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:

@@ -93,3 +93,27 @@ def test_adapter(N, device):
     # three rows of ids for two rows of tokens: unpacked ids describe no segments, as before
     odd, _ = gfa.triton_gqa_attention(mod, q, k, v, None, position_ids=torch.arange(N, device=device).repeat(3, 1))
     assert torch.equal(odd, plain)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning", "ignore::DeprecationWarning")
+@pytest.mark.parametrize("source", ["mask", "positions"])
+def test_traced_tables_follow_the_batch(source, device):
+    """Tables built inside a jit trace are part of it: they follow the batch that the trace is given,
+    not the one it was traced with."""
+    import gemma_triton_flash_attn_amd as gfa
+
+    N = 80
+    build = gfa.segments.from_padding_mask if source == "mask" else gfa.segments.from_position_ids
+    i = torch.arange(N, device=device)[None]
+
+    def batch(a, b):
+        cut = torch.tensor([[a], [b]], device=device)
+        return i < cut if source == "mask" else torch.where(i < cut, i, i - cut)
+
+    def tables(t):
+        return torch.stack(tuple(build(t)))
+
+    traced = torch.jit.trace(tables, (batch(N, 30),), check_trace=False)
+    for a, b in ((N, 30), (17, 60)):
+        same = torch.equal(traced(batch(a, b)), tables(batch(a, b)))
+        assert same, (a, b)
