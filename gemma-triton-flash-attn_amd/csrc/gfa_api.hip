@@ -165,6 +165,12 @@ bool use_rows_kernel(int D, int B, int Hq, int N, bool causal, bool windowed) {
 //   D=128 65.5 -> 58.7, 4:1 N=8192 126.3 -> 97.2; 16:4 N=2048 D=256 55.0 -> 63.9);
 // - without a mask, up to 512 blocks from 1536 tokens (8:4 N=2048 D=256 54.3 -> 51.6, D=64 24.8 -> 19.8;
 //   16:4 N=1024 D=256 30.3 -> 32.0; 576 blocks, 8:4 D=256 60.4 -> 78.0).
+// Not with a segment table, whose content the host does not know: every 32-row workgroup costs its
+// prologue and combination however short its document, so many short documents take longer (8:4
+// D=256 N=3072 in 8 / 32 documents 28.6 -> 33.0, 18.0 -> 28.3 us; N=4096 in 32 21.9 -> 36.7; 8:4 D=64
+// N=3000 in 32 9.4 -> 15.6), while rows of one or few segments would gain (N=3072 D=256 in 1 / 4
+// 79.3 -> 64.4, 56.7 -> 45.0). So a one-segment table runs another kernel than no table here,
+// and the two differ by the rounding of P against another reference maximum.
 bool use_rows_forward(int D, int B, int Hq, int N, bool causal, bool windowed, bool segments) {
   if (use_rows_kernel(D, B, Hq, N, causal, windowed)) return true;
   if (D == 512 || windowed || segments) return false;

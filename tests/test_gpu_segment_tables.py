@@ -117,3 +117,46 @@ def test_traced_tables_follow_the_batch(source, device):
     for a, b in ((N, 30), (17, 60)):
         same = torch.equal(traced(batch(a, b)), tables(batch(a, b)))
         assert same, (a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,N,D,causal,window,same", [
+    (8, 1, 333, 256, True, 512, True), (8, 1, 1024, 512, True, 0, True), (8, 1, 2500, 512, True, 0, True),
+    (8, 1, 2048, 128, True, 0, True), (8, 4, 3073, 256, True, 0, True), (4, 1, 8200, 64, True, 0, True),
+    (8, 1, 3000, 256, True, 512, True), (8, 8, 1700, 64, False, 0, False), (8, 4, 2100, 256, True, 0, False),
+    (8, 4, 3072, 256, True, 0, False), (8, 1, 4096, 128, True, 0, False), (4, 1, 8192, 64, True, 0, False),
+    (8, 4, 2048, 256, False, 0, False),
+])
+def test_ids_without_restarts(Hq, Hkv, N, D, causal, window, same, dtype, device):
+    """Position ids of one run, which a model hands over in every layer, become a table of one segment
+    per row. Outputs and gradients equal those without a table bit for bit where the same kernels
+    run (``same``); where only a call without a table takes the small-grid forward, both outputs
+    carry P rounded against their own reference maxima and their own rounding: with A = softmax
+    |V| they differ by at most 2 u (A + |O|), u = 2^-8 in bf16 and 2^-11 in fp16, plus fp32 sums
+    (1e-4)."""
+    import gemma_triton_flash_attn_amd as gfa
+
+    print(f"case {Hq}:{Hkv} N={N} D={D} causal={causal} window={window} {dtype}", flush=True)
+    g = torch.Generator(device=device).manual_seed(N)
+    q, k, v, do = (torch.randn(1, N, h, D, generator=g, device=device).to(dtype).transpose(1, 2)
+                   for h in (Hq, Hkv, Hkv, Hq))
+    mod = SimpleNamespace(head_dim=D, is_causal=causal)
+    kw = dict(sliding_window=window or None, position_ids=torch.arange(N, device=device)[None])
+    with torch.no_grad():
+        out = gfa.triton_gqa_attention(mod, q, k, v, None, **kw)[0].transpose(1, 2)
+        plain = gfa.attention_flash_gqa(q, k, v, causal, window)
+        one = gfa.segments.from_lengths([N], N, device=device)
+        assert torch.equal(out, gfa.attention_flash_gqa(q, k, v, causal, window, segments=one))
+        if not same:
+            a = gfa.attention_flash_gqa(q, k, v.abs(), causal, window)
+            u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+            assert bool(((out.float() - plain.float()).abs() <= 2 * u * (a.float() + plain.float().abs()) + 1e-4).all())
+            return
+    assert torch.equal(out, plain)
+    grads = []
+    for ids in (True, False):
+        t = [x.detach().requires_grad_(True) for x in (q, k, v)]
+        o = (gfa.triton_gqa_attention(mod, *t, None, **kw)[0].transpose(1, 2) if ids
+             else gfa.flash_attn_gqa_train(*t, causal, window))
+        grads.append(torch.autograd.grad(o, t, do))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
