@@ -9,12 +9,11 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
-#include <utility>
-#include <vector>
 
 #include "gfa.h"
 #include "gfa_launch.h"
 #include "gfa_params.h"
+#include "gfa_plan.h"
 
 namespace {
 
@@ -206,86 +205,6 @@ int pick_q_splits(int B, int Hkv, int N, int units, int wgs_per_cu, bool full_ca
 int pick_q_splits(const Entry* e, int B, int Hkv, int N, int causal, int window) {
   const DkvForm& f = dkv_form(e, causal, window, N);
   return pick_q_splits(B, Hkv, N, f.waves / f.roles, f.wgs_per_cu, causal && !is_windowed(causal, window, N));
-}
-
-// Split counts of a dK/dV grid whose key blocks are split (q_splits > 1), and its workgroups.
-//
-// q_splits equal chunks per key block keep every CU busy, but under causal masking the late blocks
-// need fewer, and every split costs fp32 partial rows: 64 keys x 512 columns of dK and dV are 256 KB
-// written and read again, so that on small grids the partials took a third of the stage. Chunks
-// of one length over the whole grid need half the splits, and one round of them ends together.
-// Which is shorter is a matter of rounding (a few chunks past one round cost a second one), so
-// the candidates are run through a list schedule of their workgroups: equal splits, and the
-// shortest common chunk that gives at most 1, 1.5 or 2 rounds. Costs in iterations (one query tile
-// of one head, 2 us at D = 512): a workgroup's prologue and epilogue take about 8, a split's
-// partials 0.03 of the whole GPU. delta + dK/dV + reduction, us, before and after: D=256 8:4
-// soft-capped N=1709 87.9 -> 66, N=3000 173 -> 132; 16:8 N=800 71 -> 47, N=1709 151 -> 90; D=512
-// 16:2 N=2048 218 -> 189; D=64 2x16:16 N=2001 50.5 -> 42; window 512 8:1 N=5000 106 -> 86.
-struct DkvPlan {
-  int chunk;
-  int nblocks;
-};  // chunk 0: equal splits
-
-DkvPlan plan_dkv(gfa::BwdDkvParams p, int wgs_per_cu) {
-  const int slots = 256 * wgs_per_cu;
-  const int copies = p.B * p.Hkv;  // grids of key blocks
-  auto iterations = [&](int kb) { return gfa::dkv_iterations(p, kb * p.wkv); };
-  auto splits = [&](int chunk, int kb) { return gfa::dkv_splits_of(iterations(kb), chunk, p.q_splits); };
-  auto count = [&](int chunk) {
-    long long c = 0;
-    for (int kb = 0; kb < p.n_kb; ++kb) c += splits(chunk, kb);
-    return c * copies;
-  };
-  // List schedule: (time, free workgroup slots) in order of time; equal workgroups move together.
-  std::vector<std::pair<int, long long>> free_at;
-  auto cost = [&](int chunk) {
-    free_at.assign(1, {0, slots});
-    int end = 0;
-    long long partials = 0;
-    for (int kb = 0; kb < p.n_kb; ++kb) {
-      const int c = splits(chunk, kb);
-      const int len = (iterations(kb) + c - 1) / c + 8;
-      long long left = (long long)c * copies;
-      if (c > 1) partials += left;
-      while (left > 0) {
-        const int t = free_at.front().first + len;
-        const long long n = std::min(left, free_at.front().second);
-        if ((free_at.front().second -= n) == 0) free_at.erase(free_at.begin());
-        auto at = std::lower_bound(free_at.begin(), free_at.end(), t, [](const auto& x, int v) { return x.first < v; });
-        if (at != free_at.end() && at->first == t) {
-          at->second += n;
-        } else {
-          free_at.insert(at, {t, n});
-        }
-        end = std::max(end, t);
-        left -= n;
-      }
-    }
-    return end + 0.03 * (double)partials;
-  };
-  int longest = 1;
-  for (int kb = 0; kb < p.n_kb; ++kb) longest = std::max(longest, iterations(kb));
-  DkvPlan best{0, (int)count(0)};
-  double best_cost = cost(0);
-  const int least = (longest + p.q_splits - 1) / p.q_splits;
-  for (int halves = 2; halves <= 4; ++halves) {
-    const long long most = (long long)slots * halves / 2;
-    int lo = least, hi = longest;  // the shortest chunk with at most `most` workgroups, or one split each
-    while (lo < hi) {
-      const int mid = (lo + hi) / 2;
-      if (count(mid) <= most) {
-        hi = mid;
-      } else {
-        lo = mid + 1;
-      }
-    }
-    const double c = cost(lo);
-    if (c < best_cost) {
-      best_cost = c;
-      best = {lo, (int)count(lo)};
-    }
-  }
-  return best;
 }
 
 gfa::RowView rv(const gfa_strides& s) { return gfa::RowView{s.batch, s.head, s.row}; }
@@ -725,8 +644,10 @@ int bwd_impl(const gfa_bwd_args* a, float* delta_buf, void* ws_buf, size_t ws_by
   if (qs > 1) {
     pk.nblocks *= qs;
     // At D=128 a CU holds up to three workgroups, which the schedule does not model: chunks only where
-    // the key blocks are few (32:8 N=1000 51.6 -> 44.2 us; N=3000, 4 splits: 198 -> 228).
-    const DkvPlan plan = a->head_dim == 128 && qs < 8 ? DkvPlan{0, 0} : plan_dkv(pk, f.wgs_per_cu);
+    // the key blocks are few (32:8 N=1000 51.6 -> 44.2 us; N=3000, 4 splits: 198 -> 228). The dQ
+    // stage alone has no dK/dV grid to plan.
+    const bool planned = (stages & GFA_BWD_DKV) && !(a->head_dim == 128 && qs < 8);
+    const gfa::DkvPlan plan = planned ? gfa::plan_dkv(pk, f.wgs_per_cu) : gfa::DkvPlan{0, 0};
     if (plan.chunk > 0) {
       pk.chunk = plan.chunk;
       pk.nblocks = plan.nblocks;

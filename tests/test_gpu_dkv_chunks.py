@@ -1,4 +1,4 @@
-"""Split dK/dV grids whose key blocks get different split counts (plan_dkv in gfa_api.hip; a block with one
+"""Split dK/dV grids whose key blocks get different split counts (plan_dkv in gfa_plan.h; a block with one
 split writes its rows directly) against the unsplit grid (q_splits = 1), on grids small enough to be
 split: every form of the kernel, ragged and odd sizes, more than 64 key blocks (the block search's
 second batch), windows, segment tables, soft-capping and dropout.
