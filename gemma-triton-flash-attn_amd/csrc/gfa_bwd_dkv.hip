@@ -24,6 +24,8 @@
 // that fed the score products. The only cross-wave traffic is the one-way P hand-off, and
 // no softmax work is duplicated. All R query heads of the KV head stream through the
 // same workgroup (pack-GQA), so K/V are read once and dK/dV need no cross-head reduction.
+#include <algorithm>
+
 #include "gfa_common.h"
 #include "gfa_params.h"
 #include "gfa_launch.h"
@@ -57,7 +59,8 @@ constexpr bool dkv_stages_rows(int D, int roles) { return roles == 1 && D >= 128
 
 // dK/dV = sum over a key block's splits of the fp32 partials, in split order, cast to the input
 // dtype; blocks with one split are written by their workgroup. One thread converts 8 consecutive
-// head-dim elements of one row; blockIdx.y is the (tensor, b, kvh) plane.
+// head-dim elements of one row, in the (tensor, b, kvh) planes blockIdx.y, + gridDim.y, ... (a grid
+// holds 65535 of them).
 template <bool IS_BF16>
 __global__ __launch_bounds__(256) void dkv_reduce_kernel(const BwdDkvParams p, int log2_d) {
   const int64_t rows = (int64_t)p.B * p.Hkv * p.N << log2_d;  // elements of one tensor
@@ -67,26 +70,28 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const BwdDkvParams p, i
   const int splits = p.chunk == 0 ? p.q_splits : dkv_splits(p, key / p.wkv * p.wkv);
   if (splits == 1) return;
   const int planes = p.B * p.Hkv;
-  const int which = blockIdx.y >= planes;
-  const int bk = blockIdx.y - which * planes;
-  const float* src = p.part + which * rows + ((int64_t)bk * p.N << log2_d) + off;
-  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int s = 0; s < splits; ++s) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(src + s * 2 * rows);
-    const f32x4 c = *reinterpret_cast<const f32x4*>(src + s * 2 * rows + 4);
+  for (int plane = blockIdx.y; plane < 2 * planes; plane += gridDim.y) {
+    const int which = plane >= planes;
+    const int bk = plane - which * planes;
+    const float* src = p.part + which * rows + ((int64_t)bk * p.N << log2_d) + off;
+    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int s = 0; s < splits; ++s) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(src + s * 2 * rows);
+      const f32x4 c = *reinterpret_cast<const f32x4*>(src + s * 2 * rows + 4);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc[e] += a[e];
-      acc[4 + e] += c[e];
+      for (int e = 0; e < 4; ++e) {
+        acc[e] += a[e];
+        acc[4 + e] += c[e];
+      }
     }
-  }
-  const RowView& v = which ? p.dvv : p.dkv;
-  uint16_t* dst = (which ? p.dv : p.dk) + (int64_t)(bk / p.Hkv) * v.sb + (int64_t)(bk % p.Hkv) * v.sh +
-                  (int64_t)key * v.sn + (off & ((1 << log2_d) - 1));
-  i16x8 o;
+    const RowView& v = which ? p.dvv : p.dkv;
+    uint16_t* dst = (which ? p.dv : p.dk) + (int64_t)(bk / p.Hkv) * v.sb + (int64_t)(bk % p.Hkv) * v.sh +
+                    (int64_t)key * v.sn + (off & ((1 << log2_d) - 1));
+    i16x8 o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = to16<IS_BF16>(acc[e]);
-  *reinterpret_cast<i16x8*>(dst) = o;
+    for (int e = 0; e < 8; ++e) o[e] = to16<IS_BF16>(acc[e]);
+    *reinterpret_cast<i16x8*>(dst) = o;
+  }
 }
 
 // Explicit instantiations of every built variant (device code and host launch stubs).
@@ -176,7 +181,7 @@ hipError_t launch_bwd_dkv(const BwdDkvParams& p, int D, int bq, int nw, int role
 hipError_t launch_dkv_reduce(const BwdDkvParams& p, int head_dim, bool bf16, hipStream_t stream) {
   const int log2_d = head_dim == 512 ? 9 : head_dim == 256 ? 8 : head_dim == 128 ? 7 : 6;
   const int64_t per_plane = ((int64_t)p.N << log2_d) / 8;
-  const dim3 grid((unsigned)((per_plane + 255) / 256), 2 * p.B * p.Hkv);
+  const dim3 grid((unsigned)((per_plane + 255) / 256), (unsigned)std::min(2 * p.B * p.Hkv, 65535));
   if (bf16) {
     hipLaunchKernelGGL(dkv_reduce_kernel<true>, grid, dim3(256), 0, stream, p, log2_d);
   } else {

@@ -64,3 +64,18 @@ def test_matches_unsplit(B, Hq, Hkv, N, D, causal, window, dtype, feature, devic
             a, b = a.float(), b.float()
             bound = ULP[dtype] * b.abs() + 1e-5 * b.abs().max()
             assert bool(((a - b).abs() <= bound).all()), (name, splits, float((a - b).abs().max()))
+
+
+def test_more_planes_than_a_grid_dimension(device):
+    """An explicit split of more (tensor, batch, KV head) planes than a launch grid's second dimension
+    holds (65535): the reduction walks them."""
+    from gemma_triton_flash_attn_amd.attention import _backward, _forward
+
+    B, N, D, dtype = 33000, 33, 128, torch.bfloat16
+    g = torch.Generator(device=device).manual_seed(1)
+    q, k, v, do = (torch.randn(B, 1, N, D, generator=g, device=device).to(dtype) for _ in range(4))
+    o, lse = _forward(q, k, v, True, 0, D ** -0.5, True)
+    got, ref = (_backward(q, k, v, o, lse, do, True, 0, D ** -0.5, q_splits=n) for n in (2, 1))
+    for a, b in zip(got[1:3], ref[1:3]):
+        a, b = a.float(), b.float()
+        assert bool(((a - b).abs() <= ULP[dtype] * b.abs() + 1e-5 * b.abs().max()).all())
