@@ -288,9 +288,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     api.last_error = pointer<decltype(api.last_error)>(last_error);
     api.error_type = error_type.release().ptr();
   });
+  // Bodies run without the interpreter lock: an allocation or a launch that waits for the driver does
+  // not hold up other Python threads (a data loader's, another stream's).
   const auto or_undefined = [](const std::optional<Tensor>& t) { return t ? *t : Tensor(); };
   // O alone, without autograd.
-  m.def("infer", torch::wrap_pybind_function(
+  m.def("infer", torch::wrap_pybind_function_no_gil(
                      [or_undefined](const Tensor& q, const Tensor& k, const Tensor& v, bool causal, int64_t window,
                                     double scale, double softcap, double dropout_p, int64_t seed, int64_t block_kv,
                                     const std::optional<Tensor>& lo, const std::optional<Tensor>& hi) {
@@ -299,7 +301,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                        return forward_call(prep(q), prep(k), prep(v), x, false).first;
                      }));
   // O with autograd.
-  m.def("train", torch::wrap_pybind_function(
+  m.def("train", torch::wrap_pybind_function_no_gil(
                      [or_undefined](const Tensor& q, const Tensor& k, const Tensor& v, bool causal, int64_t window,
                                     double scale, double softcap, double dropout_p, int64_t seed,
                                     const std::optional<Tensor>& lo, const std::optional<Tensor>& hi, bool as_op) {
@@ -308,7 +310,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                        return Attention::apply(q, k, v, x);
                      }));
   // (lo, hi) tables, int32 (batch, seq_len), of unit-stride position ids (rows of stride 0 included).
-  m.def("positions", torch::wrap_pybind_function([](const Tensor& pos) {
+  m.def("positions", torch::wrap_pybind_function_no_gil([](const Tensor& pos) {
           const c10::DeviceGuard guard(pos.device());
           const Tensor t = at::empty({2, pos.size(0), pos.size(1)}, pos.options().dtype(at::kInt));
           const Tensor lo = t.select(0, 0), hi = t.select(0, 1);

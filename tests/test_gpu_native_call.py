@@ -4,6 +4,7 @@ with saved-tensor hooks, checkpointing, function transforms, forward mode, strea
 from __future__ import annotations
 
 import threading
+import time
 from types import SimpleNamespace
 
 import pytest
@@ -181,3 +182,31 @@ def test_streams_and_threads(device):
         th.join()
     for i, (*_, want) in enumerate(cases):
         assert all(torch.equal(a, b) for a, b in zip(got[i], want))
+
+
+def test_other_threads_run_during_a_call(device):
+    """The interpreter lock is free while a call allocates (here 2 GiB from the driver) and launches:
+    another Python thread runs in the middle half of the call."""
+    import gemma_triton_flash_attn_amd as gfa
+
+    q = torch.zeros(1, 64, 131072, 128, dtype=torch.bfloat16, device=device)
+    k = q[:, :1]
+    for call in (lambda: gfa.attention_flash_gqa(q, k, k, True, 64), lambda: gfa.flash_attn_gqa_train(q, k, k, True, 64)):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        ticks, stop = [], threading.Event()
+
+        def spin():
+            while not stop.is_set():
+                ticks.append(time.perf_counter())
+
+        th = threading.Thread(target=spin)
+        th.start()
+        time.sleep(0.01)
+        t0 = time.perf_counter()
+        call()
+        t1 = time.perf_counter()
+        stop.set()
+        th.join()
+        quarter = (t1 - t0) / 4
+        assert any(t0 + quarter < t < t1 - quarter for t in ticks), t1 - t0
