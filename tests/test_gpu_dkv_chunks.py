@@ -12,7 +12,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from conftest import make_inputs
+from conftest import exact64, make_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +79,28 @@ def test_more_planes_than_a_grid_dimension(device):
     for a, b in zip(got[1:3], ref[1:3]):
         a, b = a.float(), b.float()
         assert bool(((a - b).abs() <= ULP[dtype] * b.abs() + 1e-5 * b.abs().max()).all())
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,window,dtype,feature",
+                         [c for c in CASES if c[8] in ("plain", "segments") and c[3] <= 5000])
+def test_matches_exact(B, Hq, Hkv, N, D, causal, window, dtype, feature, device):
+    """dK and dV against 64 bits, in every block of 64 keys. P, dS, O and the results are rounded to the
+    16-bit type, each within half a unit in the last place (u / 2, u = ULP / 2): independent, they
+    give about u / 2 of a block's norm, and ULP = 2 u covers it."""
+    import gemma_triton_flash_attn_amd as gfa
+    from gemma_triton_flash_attn_amd.attention import _backward, _forward
+
+    print(f"case B={B} {Hq}:{Hkv} N={N} D={D} causal={causal} window={window} {dtype} {feature}", flush=True)
+    q, k, v, do = make_inputs(B, Hq, Hkv, N, D, dtype, device, seed=N + D)
+    segs = None
+    if feature == "segments":
+        segs = gfa.segments.from_cu_seqlens([0, 1, N // 3, N // 2 + 1, N], N, device=device)
+    o, lse = _forward(q, k, v, causal, window, D ** -0.5, True, segments=segs)
+    got = _backward(q, k, v, o, lse, do, causal, window, D ** -0.5, segments=segs)
+    want = exact64(q, k, v, causal, window, segs, do)
+
+    def blocks(t):
+        return torch.nn.functional.pad(t, (0, 0, 0, -N % 64)).view(B, Hkv, -1, 64 * D).norm(dim=-1)
+
+    for name, a, b in (("dK", got[1], want[2]), ("dV", got[2], want[3])):
+        assert bool((blocks(a.double() - b) <= ULP[dtype] * blocks(b)).all()), name

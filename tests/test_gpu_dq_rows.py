@@ -13,7 +13,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from conftest import make_inputs, recomputing
+from conftest import exact64, make_inputs, recomputing
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +64,28 @@ def test_matches_recomputing(B, Hq, Hkv, N, D, causal, window, feature, dtype, d
     if feature == "segments":
         pad = (kw["segments"][0] == kw["segments"][1])[:, None, :, None].expand_as(got)
         assert bool((got[pad] == 0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,N,D,causal,window,feature",
+                         [c for c in CASES if c[7] in ("plain", "segments") and c[3] > 32])
+def test_matches_exact(B, Hq, Hkv, N, D, causal, window, feature, dtype, device):
+    """dQ against 64 bits. Its operands P, dS and O are rounded to the 16-bit type (delta = rowsum(dO O) from
+    the rounded O) and so is dQ, each rounding within u / 2 of its value; independent, they give an error of
+    about u / 2 of the norm, and 2 u covers it with room for the first rows, whose few keys add
+    nothing up."""
+    import gemma_triton_flash_attn_amd as gfa
+    from gemma_triton_flash_attn_amd.attention import _backward, _forward
+
+    print(f"case B={B} {Hq}:{Hkv} N={N} D={D} causal={causal} window={window} {dtype} {feature}", flush=True)
+    q, k, v, do = make_inputs(B, Hq, Hkv, N, D, dtype, device, seed=N + D)
+    segs = None
+    if feature == "segments":
+        rows = [gfa.segments.from_cu_seqlens([0, 1, N // 3, N // 2 + 1, N], N, device=device)]
+        rows += [gfa.segments.from_lengths([n], N, device=device) for n in (N // 2, 0, N)[:B - 1]]
+        segs = tuple(torch.cat([r[i] for r in rows]) for i in (0, 1))
+    window = 0 if window >= N else window
+    o, lse = _forward(q, k, v, causal, window, D ** -0.5, True, segments=segs)
+    got = _backward(q, k, v, o, lse, do, causal, window, D ** -0.5, segments=segs)[0]
+    want = exact64(q, k, v, causal, window, segs, do)[1]
+    assert float((got.double() - want).norm()) <= 2 * U[dtype] * float(want.norm())
