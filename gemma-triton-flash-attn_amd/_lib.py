@@ -149,13 +149,17 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+_compiling, _trace = torch.compiler.is_compiling, torch._C._get_tracing_state
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transform = torch._C._functorch.peek_interpreter_stack
+
+
 def plain_setting() -> bool:
     """Whether a call runs outside compilation, tracing, function transforms and modes (of dispatch or
     of torch functions), all of which see tensor operations and registered ops but no launch on
     their pointers."""
-    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None)
+    return (not _compiling() and _trace() is None and _dispatch_modes() == 0 and _function_modes() == 0
+            and _transform() is None)
 
 
 _native = None

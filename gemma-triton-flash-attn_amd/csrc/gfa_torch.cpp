@@ -183,14 +183,8 @@ struct Attention : public torch::autograd::Function<Attention> {
     // As the op does, a one-element CPU tensor: a compiled backward takes another seed each time.
     if (x.as_op && x.dropout_p > 0.0) saved.push_back(at::full({1}, x.seed, at::kLong));
     ctx->save_for_backward(std::move(saved));
-    ctx->saved_data["as_op"] = x.as_op;
-    ctx->saved_data["segments"] = x.lo.defined();
-    ctx->saved_data["causal"] = x.causal;
-    ctx->saved_data["window"] = x.window;
-    ctx->saved_data["scale"] = x.scale;
-    ctx->saved_data["softcap"] = x.softcap;
-    ctx->saved_data["dropout_p"] = x.dropout_p;
-    ctx->saved_data["seed"] = x.seed;
+    ctx->saved_data["whole"] = std::vector<int64_t>{x.causal, x.window, x.seed, x.as_op, x.lo.defined()};
+    ctx->saved_data["real"] = std::vector<double>{x.scale, x.softcap, x.dropout_p};
     return o;
   }
 
@@ -198,11 +192,11 @@ struct Attention : public torch::autograd::Function<Attention> {
                                                  const torch::autograd::variable_list& grads) {
     const auto saved = ctx->get_saved_variables();
     const Tensor &o = saved[3], &lse = saved[4];
-    Options x{ctx->saved_data["causal"].toBool(),      ctx->saved_data["window"].toInt(),
-              ctx->saved_data["scale"].toDouble(),     ctx->saved_data["softcap"].toDouble(),
-              ctx->saved_data["dropout_p"].toDouble(), ctx->saved_data["seed"].toInt()};
-    x.as_op = ctx->saved_data["as_op"].toBool();
-    if (ctx->saved_data["segments"].toBool()) {
+    const auto whole = ctx->saved_data["whole"].toIntVector();
+    const auto real = ctx->saved_data["real"].toDoubleVector();
+    Options x{whole[0] != 0, whole[1], real[0], real[1], real[2], whole[2]};
+    x.as_op = whole[3] != 0;
+    if (whole[4] != 0) {
       x.lo = saved[5];
       x.hi = saved[6];
     }

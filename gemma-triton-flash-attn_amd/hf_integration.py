@@ -77,8 +77,11 @@ def _segments_for(query, attention_mask, kwargs, checks=None):
         return tables
     pos = kwargs.get("position_ids")
     if pos is not None and pos.dim() == 2 and pos.shape[-1] == N:
-        on_device = pos.device == query.device and pos.shape[0] in (1, B) and seglib._native(pos)
-        if on_device or not host or seglib.is_packed(pos):
+        if pos.device == query.device and pos.shape[0] in (1, B):
+            ids = pos.expand(B, N)
+            if seglib._native(ids):
+                return seglib._from_ids(ids, True)
+        if not host or seglib.is_packed(pos):
             return seglib.from_position_ids(pos.to(query.device).expand(B, N))
     return None
 

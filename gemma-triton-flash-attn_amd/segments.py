@@ -66,8 +66,7 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
 
 
 def _new_tables(t: torch.Tensor):
-    buf = torch.empty((2, *t.shape), dtype=torch.int32, device=t.device)
-    return buf[0], buf[1]
+    return torch.empty((2, *t.shape), dtype=torch.int32, device=t.device).unbind()
 
 
 class _RunCheck:
@@ -191,7 +190,12 @@ def from_position_ids(position_ids: torch.Tensor) -> Segments:
     """Packed sequences marked by position ids (B, N): a new sequence starts wherever the
     position id is not the previous one plus one (the rule transformers uses to detect
     packed batches, masking_utils.find_packed_sequence_indices)."""
-    if position_ids.dtype in (torch.int64, torch.int32) and _native(position_ids):
+    return _from_ids(position_ids, _native(position_ids))
+
+
+def _from_ids(position_ids: torch.Tensor, native: bool) -> Segments:
+    """from_position_ids, with _native(position_ids) known."""
+    if native and position_ids.dtype in (torch.int64, torch.int32):
         return SegmentTables(*_lib.native().positions(_rows(position_ids)))
     pos = position_ids.to(torch.long)
     if pos.dim() == 1:
