@@ -221,6 +221,8 @@ def strides_of(t) -> Strides:
 
 
 def config(batch: int, heads_q: int, heads_kv: int, seq_len: int, head_dim: int) -> dict:
+    """gfa_config: the registry's tiles and split count. Grids too small to fill the GPU run 32-row
+    workgroups in the forward and in dQ from the dS store instead of the blocks reported here."""
     info = ConfigInfo()
     check(load().gfa_config(batch, heads_q, heads_kv, seq_len, head_dim, ctypes.byref(info)))
     return info.as_dict()

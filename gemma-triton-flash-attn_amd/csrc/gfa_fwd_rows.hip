@@ -18,9 +18,11 @@
 //    run most of a tile ahead of their use out of a single-buffered tile. The copies' row
 //    pieces are 256 bytes: with 128-byte ones (cells of 64 columns) the kernel took 3-6% longer at
 //    D >= 256 (8:1 D=512 N=2048 causal 70.4 -> 66.4 us, 8:4 D=256 N=700 13.9 -> 12.8 us).
-// Bound: every wave reads its own K / V from L2, 32 rows of queries per tile byte (128 in
-// fwd_kernel), so with all CUs busy the copies (64 B per CU and clock) take twice the products'
-// time. The host takes this kernel where the 128-row grid leaves CUs idle (gfa_api.hip).
+// Bound: the longest row's walk by one wave per SIMD. Every wave reads its own K / V from L2, 32 rows
+// of queries per tile byte (128 in fwd_kernel), so at best (64 B per CU and clock) the copies take
+// twice the products' time; at D=512 8:1 N=1024 a CU gets about 30 of them over the kernel (36 us
+// without a mask, 33 causal with half the bytes in all but the same longest row), matrix cores
+// 16% and 9% busy. The host takes this kernel where the 128-row grid leaves CUs idle (gfa_api.hip).
 #include "gfa_common.h"
 #include "gfa_params.h"
 #include "gfa_launch.h"

@@ -4,8 +4,8 @@
 //
 // Why: on a short sequence the kernels take 30-100 us and the host path took longer. A Python autograd
 // function's backward runs on the engine's device thread, which must first take the interpreter
-// lock from the thread that waits for it; the node here never touches the interpreter. Host time per
-// call at N=128, ctypes path against this one: forward and backward 165 -> 77 us (an elementwise
+// lock from the thread that waits for it; a plain backward here never touches the interpreter. Host
+// time per call at N=128, ctypes path against this one: forward and backward 165 -> 77 us (an elementwise
 // product's takes 59 on the same host: the rest is the engine's thread), a transformers layer
 // without gradients 55 -> 19 us, inference 16 -> 8 us.
 //
