@@ -15,6 +15,8 @@ import os
 import threading
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("GFA_LIBRARY", os.path.join(_HERE, "libgfa.so"))
@@ -157,9 +159,10 @@ _transform = torch._C._functorch.peek_interpreter_stack
 def plain_setting() -> bool:
     """Whether a call runs outside compilation, tracing, function transforms and modes (of dispatch or
     of torch functions), all of which see tensor operations and registered ops but no launch on
-    their pointers."""
-    return (not _compiling() and _trace() is None and _dispatch_modes() == 0 and _function_modes() == 0
-            and _transform() is None)
+    their pointers. A default device (torch.set_default_device, torch.device as a context) is a
+    function mode that only chooses where new tensors go, and does not count."""
+    return (not _compiling() and _trace() is None and _dispatch_modes() == 0 and _transform() is None
+            and (_function_modes() == 0 or all(type(m) is DeviceContext for m in _get_current_function_mode_stack())))
 
 
 _native = None

@@ -92,7 +92,7 @@ def padding_tables(mask: torch.Tensor):
         return from_padding_mask(mask), None
     m = _rows(mask if mask.dtype == torch.bool else mask.to(torch.bool))
     lo, hi = _new_tables(m)
-    bad = torch.empty((m.shape[0],), dtype=torch.int32, pin_memory=True)
+    bad = torch.empty((m.shape[0],), dtype=torch.int32, device="cpu", pin_memory=True)
     with torch.cuda.device(m.device):
         stream = torch.cuda.current_stream()
         _lib.check(_lib.load().gfa_segments_from_mask(m.data_ptr(), m.stride(0), m.shape[0], m.shape[1], lo.data_ptr(),

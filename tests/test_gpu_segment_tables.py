@@ -160,3 +160,31 @@ def test_ids_without_restarts(Hq, Hkv, N, D, causal, window, same, dtype, device
              else gfa.flash_attn_gqa_train(*t, causal, window))
         grads.append(torch.autograd.grad(o, t, do))
     assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
+def test_default_device(device):
+    """Under a default device (torch.set_default_device, torch.device as a context), which puts tensors made
+    without a device on the GPU, tables and calls are the same and take the same path."""
+    import gemma_triton_flash_attn_amd as gfa
+    from gemma_triton_flash_attn_amd import _lib
+
+    N = 100
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn(2, 4, N, 64, generator=g).to(device, torch.bfloat16)
+    k, v = (torch.randn(2, 2, N, 64, generator=g).to(device, torch.bfloat16) for _ in range(2))
+    mod = SimpleNamespace(head_dim=64, is_causal=True)
+    mask = (torch.arange(N)[None] < torch.tensor([[N], [40]])).to(device)
+    pos = _positions("packed", 2, N).to(device)
+
+    def calls():
+        assert _lib.plain_setting()
+        with torch.no_grad():
+            out = [gfa.triton_gqa_attention(mod, q, k, v, mask)[0],
+                   gfa.triton_gqa_attention(mod, q, k, v, None, position_ids=pos)[0],
+                   *gfa.segments.from_padding_mask(mask), *gfa.segments.from_position_ids(pos)]
+        t = [x.detach().requires_grad_(True) for x in (q, k, v)]
+        return out + list(torch.autograd.grad(gfa.triton_gqa_attention(mod, *t, mask)[0].sum(), t))
+
+    want = calls()
+    with torch.device(device):
+        assert all(torch.equal(a, b) for a, b in zip(calls(), want))
