@@ -43,10 +43,10 @@ def _segments_for(query, attention_mask, kwargs, checks=None):
       detects the same way). On the query's GPU they always become a table, of one segment per
       row where nothing restarts: one small kernel, where deciding on the host would wait for
       the device in every layer. A kernel gives the same bits, in the same time (within 1%), with
-      that table as without one, and backward and forward run the same kernels, but for the
-      forward of calls without a window at head dims 64 to 256 on few rows of heads and from 1536
-      tokens (gfa_api.hip, use_rows_forward): there only calls without a table take the faster
-      small-grid kernel (up to 1.6x), and outputs differ by the rounding of P;
+      that table as without one, and the same kernels run, but for one range: the forward
+      without a window at head dims 64 to 256, from 1536 tokens, on grids of 257 to 1024 blocks of
+      32 rows (gfa_api.hip, use_rows_forward). There only calls without a table take the
+      small-grid kernel (up to 1.6x faster), and outputs differ by the rounding of P;
     Anything else the kernels cannot express raises NotImplementedError.
 
     Under torch.compile nothing here reads device values on the host (such a read would break
