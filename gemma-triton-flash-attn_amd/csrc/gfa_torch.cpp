@@ -67,7 +67,10 @@ bool needs_copy(const Tensor& t) {
   if (((t.size(2) - 1 + kTileOverrun) * s[2] + t.size(3)) * t.element_size() > kSliceLimit) return true;
   return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 != 0;
 }
-Tensor prep(const Tensor& t) { return needs_copy(t) ? t.contiguous() : t; }
+Tensor prep(const Tensor& t) {
+  if (t.is_neg()) return prep(t.resolve_neg());  // a view that negates on reading
+  return needs_copy(t) ? t.contiguous() : t;
+}
 // An output with t's layout, or contiguous where the ABI cannot address that layout.
 Tensor out_like(const Tensor& t) {
   Tensor o = at::empty_like(t);
@@ -135,11 +138,11 @@ std::pair<Tensor, Tensor> forward_call(const Tensor& q, const Tensor& k, const T
 
 // Whether something stands between the engine and the tensors of a backward that a launch on their
 // pointers would pass by: compiled autograd's or a subclass's stand-ins for them, batched
-// gradients, a dispatch mode, a trace.
+// gradients, zeros without memory, a dispatch mode, a trace.
 bool watched(const Tensor& t) {
   using c10::DispatchKey;
   constexpr c10::DispatchKeySet keys({DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::FuncTorchBatched,
-                                      DispatchKey::FuncTorchGradWrapper, DispatchKey::Batched});
+                                      DispatchKey::FuncTorchGradWrapper, DispatchKey::Batched, DispatchKey::ZeroTensor});
   return t.key_set().has_any(keys);
 }
 bool watched(const torch::autograd::variable_list& tensors) {

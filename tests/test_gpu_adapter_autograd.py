@@ -147,3 +147,18 @@ def test_function_modes_and_profiler(grad, device):
     assert torch.equal(out, again)
     names = {e.key for e in prof.key_averages()}
     assert "gfa::attn_fwd" in names and ("gfa::attn_bwd" in names) == grad
+
+
+def test_negated_views_and_zero_gradients(device):
+    """Inputs and gradients whose values are not what lies in their memory: views that negate on reading,
+    and a zero gradient without memory."""
+    t, do = _inputs(device)
+    plain = [x.detach() for x in t]
+    neg = torch._neg_view(-plain[0])
+    assert neg.is_neg() and torch.equal(_adapter([neg, *plain[1:]], {}), _adapter(plain, {}))
+    leaves = [neg.requires_grad_(True), *t[1:]]
+    out, want = _adapter(leaves, {}), torch.autograd.grad(_op(t, {}), t, do)
+    got = torch.autograd.grad(out, leaves, torch._neg_view(-do))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    zero = torch._efficientzerotensor(do.shape, dtype=do.dtype, device=device)
+    assert all(not x.any() for x in torch.autograd.grad(_adapter(t, {}), t, zero))
